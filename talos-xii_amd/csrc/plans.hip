@@ -31,6 +31,7 @@
 #include <cstdlib>
 #include <vector>
 
+#include "acnet.hpp"
 #include "attention.hpp"
 #include "gemm.hpp"
 #include "plans.hpp"
@@ -108,6 +109,7 @@ struct talos_plan_s {
   // path instead; the same results, as the tests check at full size
   bool unfused = false;
   bool bf16 = false;  // bf16-in / fp32-accumulate GEMMs (MLA plans with TALOS_PREC_BF16)
+  double* acnet_ws = nullptr;  // the reference actor-critic runs as one kernel (acnet.hip): its partials
   bool rowdot = true;  // MLA plans: the dO product forms the attention backward's D (TALOS_MLA_ROWDOT)
   talos::Profiler* prof = nullptr;
   // latent attention: the projections before concatenation and the attention gradients,
@@ -2542,6 +2544,19 @@ int talos_ppo_plan_create(const talos_ppo_cfg* cfg, talos_plan* plan) {
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, 0) == hipSuccess) p->num_cu = prop.multiProcessorCount;
   const talos_block_cfg bc = block_cfg_of(*cfg);
+  if (!p->unfused && acnet_supported(*cfg)) {  // every activation stays in the kernel's LDS
+    float* ws = nullptr;
+    rc = upload_rope_table(p, cfg->seq, rope_width(bc), cfg->rope_base);
+    rc |= plan_alloc(p, &ws, acnet_ws_bytes(*cfg, p->num_cu) / sizeof(float));
+    p->acnet_ws = reinterpret_cast<double*>(ws);
+    if (rc) {
+      plan_free(p);
+      delete p;
+      return rc;
+    }
+    *plan = p;
+    return TALOS_OK;
+  }
   const size_t M = (size_t)cfg->batch * cfg->seq, d = cfg->d_model, B = cfg->batch, A = cfg->n_actions;
   rc = alloc_block_buffers(p, bc, cfg->n_layers);
   rc |= plan_alloc(p, &p->h0, M * d);
@@ -2604,6 +2619,19 @@ struct LensScope {
   ~LensScope() { p->lens = nullptr; }
 };
 
+// The call's common arguments of the actor-critic kernel (inside a LensScope).
+static AcNetCall acnet_call(const talos_plan_s* p, int n, const float* params, const float* states) {
+  AcNetCall a;
+  a.n = n;
+  a.params = params;
+  a.states = states;
+  a.lens = p->lens;
+  a.rcos = p->rcos;
+  a.rsin = p->rsin;
+  a.ws = p->acnet_ws;
+  return a;
+}
+
 static int ppo_check_n(const talos_plan_s* p, int n, const char* fn) {
   TALOS_REQUIRE(n >= 1 && n <= p->ppo.batch, TALOS_ERR_SHAPE, "%s: n=%d outside [1, %d] (the plan's batch)", fn, n,
                 p->ppo.batch);
@@ -2622,6 +2650,12 @@ int talos_ppo_forward_n_f32(talos_plan plan, int n, const float* params, const f
   LensScope ls(plan, lengths);
   talos_ppo_cfg c = plan->ppo;
   c.batch = n;
+  if (plan->acnet_ws) {
+    AcNetCall a = acnet_call(plan, n, params, states);
+    a.logits = logits;
+    a.values = values;
+    return entry_done(acnet_forward_launch(c, plan->num_cu, a, s), s);
+  }
   int rc = ppo_forward(plan, c, params, states, s);
   if (rc) return rc;
   if (logits)
@@ -2693,6 +2727,18 @@ static int ppo_minibatch(talos_plan_s* p, int n, const float* params, const floa
                          double* stats, int stats_acc, hipStream_t s) {
   talos_ppo_cfg c = p->ppo;
   c.batch = n;
+  if (p->acnet_ws) {
+    AcNetCall a = acnet_call(p, n, params, states);
+    a.actions = actions;
+    a.adv = adv;
+    a.ret = ret;
+    a.old_logp = old_logp;
+    a.loss = loss_out;
+    a.dparams = dparams;
+    a.stats = stats;
+    a.stats_acc = stats_acc;
+    return acnet_minibatch_launch(c, p->num_cu, a, s);
+  }
   const talos_block_cfg bc = block_cfg_of(c);
   const PpoOff po = ppo_offsets(c);
   const int M = c.batch * c.seq, d = c.d_model, A = c.n_actions, B = c.batch;
