@@ -1054,9 +1054,123 @@ __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb,
   return __builtin_bit_cast(bf16x8, u);
 }
 
+// ---------------------------------------------------------------------------
+// fp32 products on the bf16 matrix cores. Each operand value is split as it is staged into three
+// bf16 pieces, x = x0 + x1 + x2 (each the nearest bf16 to what the earlier ones left: 8 bits a piece
+// and the signs hold the 24 bits of an fp32 exactly), and a product is formed from the six pairs of
+// pieces with index sum <= 2 on v_mfma_f32_32x32x16_bf16; the three pairs left out are below 2^-26
+// of a term. x0 y0 has an accumulator of its own and the five small pairs another, added at the
+// end: with all six in one, each small product is rounded towards minus infinity at the large sum's
+// last bit, a bias that a sum over many splits of K keeps. Six 16-deep products take 192 cycles
+// where eight 2-deep fp32 ones take 512, and a K of 128 has 8 roundings at the sum's size
+// instead of 64: the error against f64 is 0.32x (K = 128) to 0.34x (K = 2048) of the fp32 chain's
+// (normal operands; 2.0e-7 -> 6.5e-8 and 8.1e-7 -> 2.8e-7 of the result's norm).
+// Values past the largest bf16 (3.39e38) and infinities have no such split: a tile whose sums are
+// not all finite is formed again by the fp32 chain. Below 2^-110 the third piece underflows: such a
+// value keeps an absolute accuracy of 2^-134.
+//
+// Panels of SK = 16 k values a stage, two stages: chunk c is multiplied while chunk c + 1 (in
+// registers, loaded two chunks earlier) is split and stored to the other stage, one barrier a
+// chunk. Piece q of a panel is a [rows][16] (k-contiguous operand) or [16][128] (k-major operand)
+// bf16 array; the 16-byte halves of row r of the first are swapped where r has bit 3 set, the
+// 16-byte pieces of k row k of the second permuted by p ^ 4 (k mod 4) as in dl_panel_kmaj, so that
+// fragment reads fall on distinct banks.
+// ---------------------------------------------------------------------------
+constexpr int SK = 16;
+// the panel [ROWS x SK] of X at rows r0, k0, as fp32 (ROWS / 64 float4s a thread): KC: thread t
+// takes k 4 (t & 3) of rows t / 4 + 64 i; else columns 4 (t & 31) of k rows t / 32 + 8 i
+template <bool KC, bool CHECK, int ROWS>
+__device__ __forceinline__ void split_load(const float* __restrict__ X, long long ld, int r0, int rlim, int k0, int kend,
+                                           bool vec, float4 (&o)[ROWS / 64]) {
+  static_assert(KC || ROWS == 128, "k-major panels have 128 columns");
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < ROWS / 64; ++i) {
+    const int r = r0 + (KC ? (t >> 2) + 64 * i : 4 * (t & 31));
+    const int k = k0 + (KC ? 4 * (t & 3) : (t >> 5) + 8 * i);
+    const float* src = KC ? X + (long long)r * ld + k : X + (long long)k * ld + r;
+    if (!CHECK || (vec && (KC ? r < rlim && k + 3 < kend : k < kend && r + 3 < rlim))) {
+      o[i] = *reinterpret_cast<const float4*>(src);
+    } else {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = (KC ? r < rlim && k + j < kend : k < kend && r + j < rlim) ? src[j] : 0.f;
+      o[i] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
+}
+// four values to their three bf16 pieces, packed
+__device__ __forceinline__ void split3(const float4& v, uint2 (&p)[3]) {
+  float r[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    p[q] = make_uint2(pack_bf16(r[0], r[1]), pack_bf16(r[2], r[3]));
+    if (q < 2) {
+      r[0] -= __uint_as_float(p[q].x << 16);
+      r[1] -= __uint_as_float(p[q].x & 0xffff0000u);
+      r[2] -= __uint_as_float(p[q].y << 16);
+      r[3] -= __uint_as_float(p[q].y & 0xffff0000u);
+    }
+  }
+}
+template <bool KC, int ROWS>
+__device__ __forceinline__ void split_store(uint16_t* S, const float4 (&v)[ROWS / 64]) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < ROWS / 64; ++i) {
+    int at;
+    if (KC) {
+      const int r = (t >> 2) + 64 * i;
+      at = r * SK + 8 * (((t >> 1) & 1) ^ ((r >> 3) & 1)) + 4 * (t & 1);
+    } else {
+      const int k = (t >> 5) + 8 * i, c = 4 * (t & 31);
+      at = k * 128 + 8 * ((c >> 3) ^ (4 * (k & 3))) + (c & 4);
+    }
+    uint2 p[3];
+    split3(v[i], p);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(S + q * ROWS * SK + at) = p[q];
+  }
+}
+// the MFMA fragment (k = 8 h + 0..7) of row / column rb + lane % 32 of one piece
+template <bool KC>
+__device__ __forceinline__ bf16x8 split_frag(const uint16_t* S, int rb, int lane) {
+  if (!KC) return dl_frag_kmaj(S, 0, rb, lane);
+  const int r = rb + (lane & 31);
+  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(S + r * SK + 8 * ((lane >> 5) ^ ((r >> 3) & 1))));
+}
+// sum (hi) and the small pairs' sum (lo) += the 16-deep product of the two stages' fragments
+template <bool KA, bool KB, int MT, int AROWS>
+__device__ __forceinline__ void split_products(const uint16_t* S, int ra, int rb, int lane, floatx16 (&hi)[MT][2],
+                                               floatx16 (&lo)[MT][2]) {
+  bf16x8 a[MT][3], b[2][3];
+  const uint16_t* Sb = S + 3 * AROWS * SK;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) b[x][q] = split_frag<KB>(Sb + q * 128 * SK, rb + 32 * x, lane);
+#pragma unroll
+    for (int x = 0; x < MT; ++x) a[x][q] = split_frag<KA>(S + q * AROWS * SK, ra + 32 * x, lane);
+  }
+  auto add = [&](int pa, int pb, floatx16 (&c)[MT][2]) {
+#pragma unroll
+    for (int x = 0; x < MT; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) c[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[x][pa], b[y][pb], c[x][y], 0, 0, 0);
+  };
+  add(0, 0, hi);
+  add(0, 1, lo);
+  add(1, 0, lo);
+  add(1, 1, lo);
+  add(0, 2, lo);
+  add(2, 0, lo);
+}
+
 template <bool TA, bool TB, int E, bool BF, int BMT>
 __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
-  __shared__ __align__(16) float smem[BF ? SMEM_BF : SMEM_FLOATS];
+  constexpr int SPLIT_STG = 3 * (BMT + BN) * SK;  // bf16 values of a stage's panels
+  constexpr int SMEM_F32 = SMEM_FLOATS > SPLIT_STG ? SMEM_FLOATS : SPLIT_STG;
+  __shared__ __align__(16) float smem[BF ? SMEM_BF : SMEM_F32];
   static_assert(BMT == 128 || (BMT == 64 && !BF), "64-row tiles are fp32 only");
   static_assert(SMEM_BF >= T_ROWS * T_S, "the staged output tile fits the bf16 panels");
   constexpr int MT = BMT / 64;  // 32-row accumulator blocks per wave
@@ -1275,50 +1389,105 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     }
   } else {
   float ssq = 0.f;  // E_NORMIN: below
-  bool direct = false;
-  // (128-row tiles: on the 64-row tiles the direct loads measured 2-5% slower at C3; one column
-  // tile: with four column tiles per row panel, N = 512 at C5, they measured 4% slower)
-  if constexpr (TALOS_GEMM_DLDS && MT == 2 && !TA && TB && (E & (E_NORMIN | E_DBIAS)) == 0) {
-    direct = interior && p.N <= BN && kbeg < kend && (kend - kbeg) % DK == 0;
-    if (direct) {
-      // stage s: the A panel (BMT rows) at smem + s (BMT + BN) DK, the B panel (BN rows) after it
-      constexpr int STG = (BMT + BN) * DK;
-      static_assert(2 * STG <= SMEM_FLOATS, "two stages fit the panels' LDS");
-      auto issue = [&](int k0, int st) {
-        dl_panel<BMT>(A, p.lda, m0, k0, smem + st * STG);
-        dl_panel<BN>(B, p.ldb, n0, k0, smem + st * STG + BMT * DK);
-      };
-      issue(kbeg, 0);
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      int st = 0;
-      for (int k0 = kbeg; k0 < kend; k0 += DK, st ^= 1) {
-        if (k0 + DK < kend) issue(k0 + DK, st ^ 1);  // the other stage was read before the last barrier
-        const float* Ap = smem + st * STG;
-        const float* Bp = Ap + BMT * DK;
-        __builtin_amdgcn_s_setprio(TALOS_GEMM_PRIO);
+  bool chain = false;  // by the fp32 chain: a sum of the split products is not finite
+  float rss[MT] = {};  // E_NORMIN: this thread's sums of squares over rows t / 4 + 64 i
+  {
+    uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
+    floatx16 lo[MT][2];
 #pragma unroll
-        for (int j = 0; j < DK / 8; ++j) {
-          float fa0[4], fa1[4], fb0[4], fb1[4];
-          dl_frag<MT == 2>(Ap, (MT == 2 ? wm * 64 : wm * 32) + l32, 8 * j + 4 * h, fa0, fa1);
-          dl_frag<true>(Bp, wn * 64 + l32, 8 * j + 4 * h, fb0, fb1);
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa0[q], fb0[q], acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa0[q], fb1[q], acc[0][1], 0, 0, 0);
-            if constexpr (MT == 2) {
-              acc[MT - 1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa1[q], fb0[q], acc[MT - 1][0], 0, 0, 0);
-              acc[MT - 1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa1[q], fb1[q], acc[MT - 1][1], 0, 0, 0);
-            }
-          }
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) lo[i][j][r] = 0.f;
+    float4 cs4 = make_float4(0.f, 0.f, 0.f, 0.f);  // E_DBIAS: column sums over the thread's k rows
+    struct Regs {
+      float4 a[MT], b[2];
+    };
+    auto load = [&](int k0, Regs& R) {
+      if (interior && k0 + SK <= kend) {
+        split_load<!TA, false, BMT>(A, p.lda, m0, p.M, k0, kend, true, R.a);
+        split_load<TB, false, BN>(B, p.ldb, n0, p.N, k0, kend, true, R.b);
+      } else {
+        split_load<!TA, true, BMT>(A, p.lda, m0, p.M, k0, kend, p.vecA, R.a);
+        split_load<TB, true, BN>(B, p.ldb, n0, p.N, k0, kend, p.vecB, R.b);
+      }
+    };
+    auto store = [&](int k0, int st, Regs& R) {
+      if constexpr ((E & E_DBIAS) != 0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          cs4.x += R.b[i].x;
+          cs4.y += R.b[i].y;
+          cs4.z += R.b[i].z;
+          cs4.w += R.b[i].w;
         }
-        __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the next chunk have landed
-        __syncthreads();                // everyone's, and every wave is done with this stage
+      }
+      if constexpr ((E & E_NORMIN) != 0) {
+        static_assert(!TA && !TB && BMT == 128, "input norm: A and B plain, 128-row tiles");
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          rss[i] += R.a[i].x * R.a[i].x + R.a[i].y * R.a[i].y + R.a[i].z * R.a[i].z + R.a[i].w * R.a[i].w;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int k = k0 + (threadIdx.x >> 5) + 8 * i;
+          const float g = k < kend ? p.nin_gain[k] : 0.f;
+          R.b[i] = make_float4(R.b[i].x * g, R.b[i].y * g, R.b[i].z * g, R.b[i].w * g);
+        }
+      }
+      split_store<!TA, BMT>(S16 + st * SPLIT_STG, R.a);
+      split_store<TB, BN>(S16 + st * SPLIT_STG + 3 * BMT * SK, R.b);
+    };
+    // chunk k0 from stage st; R holds chunk k0 + SK and takes chunk k0 + 3 SK
+    auto step = [&](int k0, int st, Regs& R) {
+      split_products<!TA, TB, MT, BMT>(S16 + st * SPLIT_STG, wm * (BMT / 2), wn * 64, lane, acc, lo);
+      if (k0 + SK < kend) {
+        store(k0 + SK, st ^ 1, R);
+        if (k0 + 3 * SK < kend) load(k0 + 3 * SK, R);
+      }
+      lds_barrier();
+    };
+    Regs r0, r1;
+    if (kbeg < kend) {
+      load(kbeg, r0);
+      if (kbeg + SK < kend) load(kbeg + SK, r1);
+      store(kbeg, 0, r0);
+      if (kbeg + 2 * SK < kend) load(kbeg + 2 * SK, r0);
+    }
+    lds_barrier();
+    for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
+      step(k0, 0, r1);
+      if (k0 + SK < kend) step(k0 + SK, 1, r0);
+    }
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[i][j][r] += lo[i][j][r];
+          bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
+        }
+    chain = __syncthreads_or(bad);
+    if constexpr ((E & E_DBIAS) != 0) {
+      // the eight row groups' sums of each column, added below as the chain's two halves are
+      if (m0 == 0 && !chain) {
+        *reinterpret_cast<float4*>(smem + (threadIdx.x >> 5) * BN + 4 * (threadIdx.x & 31)) = cs4;
+        __syncthreads();
+        const float* c = smem + (threadIdx.x & 127) + (threadIdx.x >> 7) * 4 * BN;
+        csum = (c[0] + c[BN]) + (c[2 * BN] + c[3 * BN]);
+        __syncthreads();
       }
     }
   }
-  if (!direct) {
+  if (chain) {
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   float4 ra[BMT / 32], rb[4];
   // E_NORMIN: this thread's sum of squares over the A values it loads (thread t and t + 128 load
   // the halves of tile row t % 128), and the gain applied to the B rows as they are loaded
@@ -1400,12 +1569,23 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     }
   }
   if (NBUF == 2 || kbeg >= kend) __syncthreads();
-  }  // !direct
+  }  // chain
   if constexpr ((E & E_NORMIN) != 0) {
     // rstd of each tile row, the accumulators scaled by their row's, and (first column tile) the
     // normalised rows and rstd written out
     __shared__ float nin_rs[BMT];
-    smem[threadIdx.x] = ssq;
+    if (chain) {
+      smem[threadIdx.x] = ssq;
+    } else {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        float v = rss[i];
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        if ((threadIdx.x & 3) == 0) smem[(threadIdx.x >> 2) + 64 * i] = v;
+        if ((threadIdx.x & 3) == 1) smem[BMT + (threadIdx.x >> 2) + 64 * i] = 0.f;
+      }
+    }
     __syncthreads();
     if (threadIdx.x < BMT)
       nin_rs[threadIdx.x] = 1.0f / sqrtf((smem[threadIdx.x] + smem[threadIdx.x + BMT]) / (float)p.K + p.nin_eps);
@@ -1646,7 +1826,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
 }
 
 template <bool TA, bool TB, int E, bool BF>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(BF ? 2 : TALOS_GEMM_WAVES))) void gemm_f32_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f32_kernel(
     GemmArgs p) {
   const int logical = xcd_logical();
   if (logical >= p.nblocks) return;
@@ -1656,7 +1836,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(BF ? 2 : TAL
 // 64 x 128 tiles for the products whose 128 x 128 tiles would leave each CU fewer than two
 // workgroups (d = 128 outputs over 32K rows): twice the workgroups, half the serial chain each.
 template <bool TA, bool TB, int E>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(TALOS_GEMM_WAVES))) void gemm_f32_m64_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void gemm_f32_m64_kernel(
     GemmArgs p) {
   const int logical = xcd_logical();
   if (logical >= p.nblocks) return;
@@ -1668,7 +1848,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(TALOS_GEMM_W
 // some left, then the larger one takes the rest, so every XCD runs both products in contiguous
 // runs of each. Four workgroups per CU where each product alone would give two.
 template <bool TA, bool TB, int E>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(TALOS_GEMM_WAVES))) void gemm_f32_pair_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_f32_pair_kernel(
     GemmArgs p0, GemmArgs p1) {
   const int logical = xcd_logical();
   const int m = min(p0.nblocks, p1.nblocks);
