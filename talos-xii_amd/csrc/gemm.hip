@@ -1414,24 +1414,26 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
       }
     };
     auto store = [&](int k0, int st, Regs& R) {
+      const bool in = k0 < kend;  // (uniform; past kend the registers hold nothing of the product)
       if constexpr ((E & E_DBIAS) != 0) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          cs4.x += R.b[i].x;
-          cs4.y += R.b[i].y;
-          cs4.z += R.b[i].z;
-          cs4.w += R.b[i].w;
+          cs4.x += in ? R.b[i].x : 0.f;
+          cs4.y += in ? R.b[i].y : 0.f;
+          cs4.z += in ? R.b[i].z : 0.f;
+          cs4.w += in ? R.b[i].w : 0.f;
         }
       }
       if constexpr ((E & E_NORMIN) != 0) {
         static_assert(!TA && !TB && BMT == 128, "input norm: A and B plain, 128-row tiles");
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-          rss[i] += R.a[i].x * R.a[i].x + R.a[i].y * R.a[i].y + R.a[i].z * R.a[i].z + R.a[i].w * R.a[i].w;
+        for (int i = 0; i < MT; ++i) {
+          const float ss = R.a[i].x * R.a[i].x + R.a[i].y * R.a[i].y + R.a[i].z * R.a[i].z + R.a[i].w * R.a[i].w;
+          rss[i] += in ? ss : 0.f;
+        }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int k = k0 + (threadIdx.x >> 5) + 8 * i;
-          const float g = k < kend ? p.nin_gain[k] : 0.f;
+        for (int i = 0; i < 2; ++i) {  // (rows past kend hold zeros or are not read)
+          const float g = p.nin_gain[min(k0 + (int)(threadIdx.x >> 5) + 8 * i, kend - 1)];
           R.b[i] = make_float4(R.b[i].x * g, R.b[i].y * g, R.b[i].z * g, R.b[i].w * g);
         }
       }
@@ -1455,9 +1457,28 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
       if (kbeg + 2 * SK < kend) load(kbeg + 2 * SK, r0);
     }
     lds_barrier();
-    for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
-      step(k0, 0, r1);
-      if (k0 + SK < kend) step(k0 + SK, 1, r0);
+    if (interior && kbeg < kend && (kend - kbeg) % (2 * SK) == 0) {
+      // whole chunks, an even number: no branch inside a step, so that the split of the next chunk
+      // and its stores can be issued between the products (a branch there made a wave walk its
+      // products, then its split: 2430 cycles a chunk against the products' 1536 for two waves a
+      // SIMD). The last steps split and store registers nobody reads and load the last chunk again.
+      auto fast = [&](int k0, int st, Regs& R) {
+        split_products<!TA, TB, MT, BMT>(S16 + st * SPLIT_STG, wm * (BMT / 2), wn * 64, lane, acc, lo);
+        store(k0 + SK, st ^ 1, R);
+        const int kn = min(k0 + 3 * SK, kend - SK);
+        split_load<!TA, false, BMT>(A, p.lda, m0, p.M, kn, kend, true, R.a);
+        split_load<TB, false, BN>(B, p.ldb, n0, p.N, kn, kend, true, R.b);
+        lds_barrier();
+      };
+      for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
+        fast(k0, 0, r1);
+        fast(k0 + SK, 1, r0);
+      }
+    } else {
+      for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
+        step(k0, 0, r1);
+        if (k0 + SK < kend) step(k0 + SK, 1, r0);
+      }
     }
     bool bad = false;
 #pragma unroll
@@ -1469,15 +1490,19 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
           acc[i][j][r] += lo[i][j][r];
           bad |= !(fabsf(acc[i][j][r]) <= 3.402823466e38f);
         }
-    chain = __syncthreads_or(bad);
+    __shared__ int bad_wave[4];
+    if (lane == 0) bad_wave[w] = 0;
+    if (__any(bad) && lane == 0) bad_wave[w] = 1;
+    lds_barrier();
+    chain = (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
     if constexpr ((E & E_DBIAS) != 0) {
       // the eight row groups' sums of each column, added below as the chain's two halves are
       if (m0 == 0 && !chain) {
         *reinterpret_cast<float4*>(smem + (threadIdx.x >> 5) * BN + 4 * (threadIdx.x & 31)) = cs4;
-        __syncthreads();
+        lds_barrier();
         const float* c = smem + (threadIdx.x & 127) + (threadIdx.x >> 7) * 4 * BN;
         csum = (c[0] + c[BN]) + (c[2 * BN] + c[3 * BN]);
-        __syncthreads();
+        lds_barrier();
       }
     }
   }
@@ -1691,7 +1716,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
   if constexpr (NB_PIPE) {
     constexpr bool LAST = (E & E_NBLAST) != 0;
     stage_acc<MT>(T, acc, wm, wn, h, l32, 0);
-    __syncthreads();
+    lds_barrier();
     // (each thread reads and writes only its own rows' columns of T from here on)
     if constexpr ((E & E_NBPRE) != 0) normb_pre_rows(p, T, cg, col, m0 + (threadIdx.x >> 5));
     const float4 g = *reinterpret_cast<const float4*>(p.nb_gain + col);
@@ -1699,7 +1724,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
   }
 #pragma unroll
   for (int half = 0; half < (NB_PIPE ? 0 : BMT / T_ROWS); ++half) {
-    if (half) __syncthreads();  // the first half has been read out
+    if (half) lds_barrier();  // the first half has been read out
     if (MT == 1 || wm == half) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
@@ -1712,7 +1737,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
             T[row * T_S + c] = acc[mt][nt][r];
           }
     }
-    __syncthreads();
+    lds_barrier();
     if constexpr ((E & E_SPLIT) != 0) {
       float* P = p.part + ((long long)b * p.ksplit + split) * (long long)(p.M + ((E & E_DBIAS) ? 1 : 0)) * p.N;
       const bool vec_out = (p.N & 3) == 0;
@@ -1813,9 +1838,9 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
   }
   if constexpr ((E & E_NORMB) != 0) {
     // the tile's dgain partial: the 8 row groups' sums of each column added in f64, in order
-    __syncthreads();  // T has been read out
+    lds_barrier();  // T has been read out
     *reinterpret_cast<float4*>(T + (threadIdx.x >> 5) * BN + cg) = nbw;
-    __syncthreads();
+    lds_barrier();
     if (threadIdx.x < BN) {
       double sum = 0.0;
 #pragma unroll
