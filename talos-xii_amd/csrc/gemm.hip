@@ -1040,15 +1040,17 @@ __device__ __forceinline__ void lds_barrier() {
 // ds_read_b64_tr_b16. That instruction works on groups of 16 lanes: lane 4a + j of a group gives
 // the address of four consecutive values (row a of a 4 x 16 block, columns 4j .. 4j + 3) and lane
 // l receives column l of the block's four rows. Group g = lane / 16 takes columns cb + 16 (g mod 2)
-// .. + 15 of k rows 16 s + 8 (g / 2) + 0..3, then + 4..7.
+// .. + 15 of k rows 16 s + 8 (g / 2) + 0..3, then + 4..7. (COLS = 64: rows two apart share banks, so
+// piece p of k row r sits in slot p ^ 2 (r & 2).)
+template <int COLS = 128>
 __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb, int lane) {
   typedef short shortx4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) shortx4* lds_x4;
   const int g = lane >> 4, a = (lane >> 2) & 3, j = lane & 3;
   const int k = 16 * s + 8 * (g >> 1) + a, pc = (cb >> 3) + 2 * (g & 1) + (j >> 1);
-  const uint16_t* q = S + k * 128 + 8 * (pc ^ (4 * a)) + 4 * (j & 1);  // k mod 4 = a
+  const uint16_t* q = S + k * COLS + 8 * (pc ^ (COLS == 128 ? 4 * a : 2 * (a & 2))) + 4 * (j & 1);  // k mod 4 = a
   const shortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_x4)(q));
-  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_x4)(q + 4 * 128));
+  const shortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_x4)(q + 4 * COLS));
   const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
   const uint4 u = {l2.x, l2.y, h2.x, h2.y};
   return __builtin_bit_cast(bf16x8, u);
@@ -1078,16 +1080,16 @@ __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb,
 // ---------------------------------------------------------------------------
 constexpr int SK = 16;
 // the panel [ROWS x SK] of X at rows r0, k0, as fp32 (ROWS / 64 float4s a thread): KC: thread t
-// takes k 4 (t & 3) of rows t / 4 + 64 i; else columns 4 (t & 31) of k rows t / 32 + 8 i
+// takes k 4 (t & 3) of rows t / 4 + 64 i; else columns 4 (t mod L) of k rows t / L + 8 i (L = ROWS / 4)
 template <bool KC, bool CHECK, int ROWS>
 __device__ __forceinline__ void split_load(const float* __restrict__ X, long long ld, int r0, int rlim, int k0, int kend,
                                            bool vec, float4 (&o)[ROWS / 64]) {
-  static_assert(KC || ROWS == 128, "k-major panels have 128 columns");
+  constexpr int L = ROWS / 4;  // lanes a k row of a k-major panel
   const int t = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < ROWS / 64; ++i) {
-    const int r = r0 + (KC ? (t >> 2) + 64 * i : 4 * (t & 31));
-    const int k = k0 + (KC ? 4 * (t & 3) : (t >> 5) + 8 * i);
+    const int r = r0 + (KC ? (t >> 2) + 64 * i : 4 * (t % L));
+    const int k = k0 + (KC ? 4 * (t & 3) : t / L + 8 * i);
     const float* src = KC ? X + (long long)r * ld + k : X + (long long)k * ld + r;
     if (!CHECK || (vec && (KC ? r < rlim && k + 3 < kend : k < kend && r + 3 < rlim))) {
       o[i] = *reinterpret_cast<const float4*>(src);
@@ -1123,8 +1125,8 @@ __device__ __forceinline__ void split_store(uint16_t* S, const float4 (&v)[ROWS 
       const int r = (t >> 2) + 64 * i;
       at = r * SK + 8 * (((t >> 1) & 1) ^ ((r >> 3) & 1)) + 4 * (t & 1);
     } else {
-      const int k = (t >> 5) + 8 * i, c = 4 * (t & 31);
-      at = k * 128 + 8 * ((c >> 3) ^ (4 * (k & 3))) + (c & 4);
+      const int k = t / (ROWS / 4) + 8 * i, c = 4 * (t % (ROWS / 4));
+      at = k * ROWS + 8 * ((c >> 3) ^ (ROWS == 128 ? 4 * (k & 3) : 2 * (k & 2))) + (c & 4);
     }
     uint2 p[3];
     split3(v[i], p);
@@ -1133,9 +1135,9 @@ __device__ __forceinline__ void split_store(uint16_t* S, const float4 (&v)[ROWS 
   }
 }
 // the MFMA fragment (k = 8 h + 0..7) of row / column rb + lane % 32 of one piece
-template <bool KC>
+template <bool KC, int COLS = 128>
 __device__ __forceinline__ bf16x8 split_frag(const uint16_t* S, int rb, int lane) {
-  if (!KC) return dl_frag_kmaj(S, 0, rb, lane);
+  if (!KC) return dl_frag_kmaj<COLS>(S, 0, rb, lane);
   const int r = rb + (lane & 31);
   return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(S + r * SK + 8 * ((lane >> 5) ^ ((r >> 3) & 1))));
 }
@@ -1450,31 +1452,43 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
       lds_barrier();
     };
     Regs r0, r1;
-    if (kbeg < kend) {
-      load(kbeg, r0);
-      if (kbeg + SK < kend) load(kbeg + SK, r1);
-      store(kbeg, 0, r0);
-      if (kbeg + 2 * SK < kend) load(kbeg + 2 * SK, r0);
-    }
-    lds_barrier();
     if (interior && kbeg < kend && (kend - kbeg) % (2 * SK) == 0) {
-      // whole chunks, an even number: no branch inside a step, so that the split of the next chunk
-      // and its stores can be issued between the products (a branch there made a wave walk its
-      // products, then its split: 2430 cycles a chunk against the products' 1536 for two waves a
-      // SIMD). The last steps split and store registers nobody reads and load the last chunk again.
+      // whole chunks, an even number: no branch inside a step, so that the split of the next chunk and its stores can
+      // be issued between the products (a branch there made a wave walk its products, then its
+      // split: 2430 cycles a chunk against the products' 1536 for two waves a SIMD), nor around the
+      // first loads (the wait before a split would then drain the loads issued after its own). The
+      // last steps split and store registers nobody reads and load the last chunk again.
+      auto fetch = [&](int k0, Regs& R) {
+        const int kn = min(k0, kend - SK);
+        split_load<!TA, false, BMT>(A, p.lda, m0, p.M, kn, kend, true, R.a);
+        split_load<TB, false, BN>(B, p.ldb, n0, p.N, kn, kend, true, R.b);
+      };
       auto fast = [&](int k0, int st, Regs& R) {
         split_products<!TA, TB, MT, BMT>(S16 + st * SPLIT_STG, wm * (BMT / 2), wn * 64, lane, acc, lo);
         store(k0 + SK, st ^ 1, R);
-        const int kn = min(k0 + 3 * SK, kend - SK);
-        split_load<!TA, false, BMT>(A, p.lda, m0, p.M, kn, kend, true, R.a);
-        split_load<TB, false, BN>(B, p.ldb, n0, p.N, kn, kend, true, R.b);
+        fetch(k0 + 3 * SK, R);
         lds_barrier();
       };
+      // (in this order: the wait for r1 at the head of the loop is set for its loads being older)
+      fetch(kbeg, r0);
+      asm volatile("" ::: "memory");
+      fetch(kbeg + SK, r1);
+      asm volatile("" ::: "memory");
+      store(kbeg, 0, r0);
+      fetch(kbeg + 2 * SK, r0);
+      lds_barrier();
       for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
         fast(k0, 0, r1);
         fast(k0 + SK, 1, r0);
       }
     } else {
+      if (kbeg < kend) {
+        load(kbeg, r0);
+        if (kbeg + SK < kend) load(kbeg + SK, r1);
+        store(kbeg, 0, r0);
+        if (kbeg + 2 * SK < kend) load(kbeg + 2 * SK, r0);
+      }
+      lds_barrier();
       for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
         step(k0, 0, r1);
         if (k0 + SK < kend) step(k0 + SK, 1, r0);
@@ -1903,7 +1917,8 @@ constexpr int SBM = 64, SBN = 64;
 constexpr int S_LDS = 72;
 constexpr int S_PANEL = (BK * S_LDS > SBM * KP) ? BK * S_LDS : SBM * KP;
 constexpr int S_TS = 72;  // staged output tile pitch (the half-wave rows 4 apart: 32 banks apart)
-constexpr int S_SMEM = (2 * S_PANEL > SBM * S_TS) ? 2 * S_PANEL : SBM * S_TS;
+constexpr int S_SMEM0 = (2 * S_PANEL > SBM * S_TS) ? 2 * S_PANEL : SBM * S_TS;
+constexpr int S_SMEM = S_SMEM0 > 3 * (SBM + SBN) * SK ? S_SMEM0 : 3 * (SBM + SBN) * SK;  // (two stages of split panels)
 
 // op(X) panel [64 rows x 32 k] of chunk k0 into registers. KC: X[r][k] (k contiguous), thread t
 // takes row t%64, k = 4*(t/64 + 4i); otherwise X[k][r] (r contiguous), thread t takes
@@ -1961,7 +1976,7 @@ __device__ __forceinline__ void s_frag(const float* X, int r, int k0, float (&f)
 }
 
 template <bool TA, bool TB, int E>
-__global__ __launch_bounds__(NT) void gemm_small_kernel(GemmArgs p) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gemm_small_kernel(GemmArgs p) {
   __shared__ __align__(16) float smem[S_SMEM];
   float* const As = smem;
   float* const Bs = smem + S_PANEL;
@@ -1988,6 +2003,123 @@ __global__ __launch_bounds__(NT) void gemm_small_kernel(GemmArgs p) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float csum = 0.f;  // E_DBIAS: column t%64 of op(B) over rows 8*(t/64) .. +8 of each panel
+  bool chain = false;
+  {  // the split products (gemm_tile's, a 32 x 32 block a wave)
+    constexpr int STG = 3 * (SBM + SBN) * SK;
+    uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
+    floatx16 lo, lo1;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) lo[r] = lo1[r] = 0.f;
+    float4 cs4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    struct Regs {
+      float4 a[1], b[1];
+    };
+    auto load = [&](int k0, Regs& R) {
+      if (interior && k0 + SK <= kend) {
+        split_load<!TA, false, SBM>(A, p.lda, m0, p.M, k0, kend, true, R.a);
+        split_load<TB, false, SBN>(B, p.ldb, n0, p.N, k0, kend, true, R.b);
+      } else {
+        split_load<!TA, true, SBM>(A, p.lda, m0, p.M, k0, kend, p.vecA, R.a);
+        split_load<TB, true, SBN>(B, p.ldb, n0, p.N, k0, kend, p.vecB, R.b);
+      }
+    };
+    auto store = [&](int k0, int st, Regs& R) {
+      if constexpr ((E & E_DBIAS) != 0) {
+        const bool in = k0 < kend;
+        cs4.x += in ? R.b[0].x : 0.f;
+        cs4.y += in ? R.b[0].y : 0.f;
+        cs4.z += in ? R.b[0].z : 0.f;
+        cs4.w += in ? R.b[0].w : 0.f;
+      }
+      split_store<!TA, SBM>(S16 + st * STG, R.a);
+      split_store<TB, SBN>(S16 + st * STG + 3 * SBM * SK, R.b);
+    };
+    auto products = [&](int st) {
+      bf16x8 fa[3], fb[3];
+      const uint16_t* S = S16 + st * STG;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        fa[q] = split_frag<!TA, SBM>(S + q * SBM * SK, wm * 32, lane);
+        fb[q] = split_frag<TB, SBN>(S + (3 * SBM + q * SBN) * SK, wn * 32, lane);
+      }
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[1], lo, 0, 0, 0);
+      lo1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1], fb[0], lo1, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[0], acc, 0, 0, 0);
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1], fb[1], lo, 0, 0, 0);
+      lo1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[2], lo1, 0, 0, 0);
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[2], fb[0], lo, 0, 0, 0);
+    };
+    Regs r0, r1;
+    if (interior && kbeg < kend && (kend - kbeg) % (2 * SK) == 0) {
+      auto fetch = [&](int k0, Regs& R) {
+        const int kn = min(k0, kend - SK);
+        split_load<!TA, false, SBM>(A, p.lda, m0, p.M, kn, kend, true, R.a);
+        split_load<TB, false, SBN>(B, p.ldb, n0, p.N, kn, kend, true, R.b);
+      };
+      auto fast = [&](int k0, int st, Regs& R) {
+        products(st);
+        store(k0 + SK, st ^ 1, R);
+        fetch(k0 + 3 * SK, R);
+        lds_barrier();
+      };
+      fetch(kbeg, r0);
+      asm volatile("" ::: "memory");  // (in this order, as in gemm_tile)
+      fetch(kbeg + SK, r1);
+      asm volatile("" ::: "memory");
+      store(kbeg, 0, r0);
+      fetch(kbeg + 2 * SK, r0);
+      lds_barrier();
+      for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
+        fast(k0, 0, r1);
+        fast(k0 + SK, 1, r0);
+      }
+    } else {
+      auto step = [&](int k0, int st, Regs& R) {
+        products(st);
+        if (k0 + SK < kend) {
+          store(k0 + SK, st ^ 1, R);
+          if (k0 + 3 * SK < kend) load(k0 + 3 * SK, R);
+        }
+        lds_barrier();
+      };
+      if (kbeg < kend) {
+        load(kbeg, r0);
+        if (kbeg + SK < kend) load(kbeg + SK, r1);
+        store(kbeg, 0, r0);
+        if (kbeg + 2 * SK < kend) load(kbeg + 2 * SK, r0);
+      }
+      lds_barrier();
+      for (int k0 = kbeg; k0 < kend; k0 += 2 * SK) {
+        step(k0, 0, r1);
+        if (k0 + SK < kend) step(k0 + SK, 1, r0);
+      }
+    }
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc[r] += lo[r] + lo1[r];
+      bad |= !(fabsf(acc[r]) <= 3.402823466e38f);
+    }
+    __shared__ int bad_wave[4];
+    if (lane == 0) bad_wave[w] = 0;
+    if (__any(bad) && lane == 0) bad_wave[w] = 1;
+    if constexpr ((E & E_DBIAS) != 0)
+      if (m0 == 0) *reinterpret_cast<float4*>(smem + (threadIdx.x >> 4) * SBN + 4 * (threadIdx.x & 15)) = cs4;
+    lds_barrier();
+    chain = (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
+    if constexpr ((E & E_DBIAS) != 0) {
+      // the sixteen k rows' sums of each column, four to a thread, added below as the chain's
+      // quarters are
+      if (m0 == 0 && !chain) {
+        const float* c = smem + (threadIdx.x & 63) + (threadIdx.x >> 6) * 4 * SBN;
+        csum = (c[0] + c[SBN]) + (c[2 * SBN] + c[3 * SBN]);
+      }
+      lds_barrier();
+    }
+  }
+  if (chain) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float4 ra[2], rb[2];
   auto load = [&](int k0) {
     if (interior && k0 + BK <= kend) {
@@ -2029,6 +2161,7 @@ __global__ __launch_bounds__(NT) void gemm_small_kernel(GemmArgs p) {
       __syncthreads();
     }
   }
+  }  // chain
   if constexpr ((E & E_DBIAS) != 0) {
     if (m0 == 0) {
       smem[threadIdx.x] = csum;
@@ -2266,12 +2399,13 @@ static int epi_flags(const GemmDesc& d) {
 // and split K instead, which reads each operand half as often.
 static void (*pick_m64(bool tA, bool tB, int e))(GemmArgs);
 // The 64 x 64 tile kernel for products of fewer 128 x 128 tiles than CUs and at most 2^30 MACs;
-// not for one 128-wide column of tiles over at least 64 rows a CU where the 64 x 128 tiles are
-// instantiated (C5's M = 16384, N = 128 products: 1.669 -> 1.650 ms).
+// not for one 128-wide column of tiles over at least 40 rows a CU where the 64 x 128 tiles are
+// instantiated: these split half as many operand values a product, and their norm epilogues save
+// the row kernels (14700 x 128 x 512: 230 workgroups, about one a CU, against 460).
 static bool use_small(const GemmDesc& d, int num_cu) {
   const long long tiles = (long long)((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN) * d.batch;
   const double macs = (double)d.M * d.N * d.K * d.batch;
-  if (!d.bf16 && d.batch == 1 && d.N <= BN && d.M >= 64 * num_cu && !d.transA && d.ksplit <= 1 &&
+  if (!d.bf16 && d.batch == 1 && d.N <= BN && d.N > SBN && d.M >= 40 * num_cu && !d.transA && d.ksplit <= 1 &&
       pick_m64(false, d.transB != 0, epi_flags(d)) != nullptr)
     return false;  // one 128-wide column of tiles over many rows: the 64-row tiles
   return !d.bf16 && d.cmap_w == 0 && !d.rd_D && tiles < num_cu && macs <= 1073741824.0;
