@@ -2007,9 +2007,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
   {  // the split products (gemm_tile's, a 32 x 32 block a wave)
     constexpr int STG = 3 * (SBM + SBN) * SK;
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
-    floatx16 lo, lo1;
+    floatx16 lo;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) lo[r] = lo1[r] = 0.f;
+    for (int r = 0; r < 16; ++r) lo[r] = 0.f;
     float4 cs4 = make_float4(0.f, 0.f, 0.f, 0.f);
     struct Regs {
       float4 a[1], b[1];
@@ -2042,11 +2042,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
         fa[q] = split_frag<!TA, SBM>(S + q * SBM * SK, wm * 32, lane);
         fb[q] = split_frag<TB, SBN>(S + (3 * SBM + q * SBN) * SK, wn * 32, lane);
       }
-      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[1], lo, 0, 0, 0);
-      lo1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1], fb[0], lo1, 0, 0, 0);
+      // (split_products' order, so that a product has the same bits on either tile size)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[0], acc, 0, 0, 0);
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[1], lo, 0, 0, 0);
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1], fb[0], lo, 0, 0, 0);
       lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1], fb[1], lo, 0, 0, 0);
-      lo1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[2], lo1, 0, 0, 0);
+      lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[2], lo, 0, 0, 0);
       lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[2], fb[0], lo, 0, 0, 0);
     };
     Regs r0, r1;
@@ -2097,7 +2098,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
     bool bad = false;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      acc[r] += lo[r] + lo1[r];
+      acc[r] += lo[r];
       bad |= !(fabsf(acc[r]) <= 3.402823466e38f);
     }
     __shared__ int bad_wave[4];
