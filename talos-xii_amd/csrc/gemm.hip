@@ -469,21 +469,8 @@ __device__ __forceinline__ void epi_norm4(const GemmArgs& p, float4 o, int row, 
 // norm's output; the 32 lanes of a half-wave hold one row): dx = rstd * (gg * gain - x_hat * md)
 // + the addends, md = mean(gg * gain * x_hat), x_hat = x * rstd; the lane's dgain terms gg * x_hat
 // are added to dw (column group col). Same arithmetic as rmsnorm_bwd_kernel. Every lane of the
-// half-wave takes part in the shuffle; rows past M contribute zeros. The row's x and rstd are
-// loaded by normb_load one row ahead (normb_apply uses them), so the epilogue's loads overlap the
-// previous row's work instead of each row waiting on memory.
-struct NbIn {
-  float4 x;
-  float r;
-};
-__device__ __forceinline__ NbIn normb_load(const GemmArgs& p, int row, int col) {
-  NbIn in;
-  const bool on = row < p.M;
-  in.r = on ? p.nb_rstd[row] : 0.f;
-  in.x = on ? *reinterpret_cast<const float4*>(p.nb_x + (long long)row * p.N + col) : make_float4(0.f, 0.f, 0.f, 0.f);
-  return in;
-}
-// Every operand of one row of the pipelined norm-backward epilogue (64-row tiles, E_NORMB without E_NBPRE),
+// half-wave takes part in the shuffle; rows past M contribute zeros.
+// Every operand of one row of the norm-backward epilogue,
 // loaded kNbAhead rows ahead of its use with no branch around a load: the last-row addends are
 // read for every row (a clamped, valid row) and kept only for the sample's last row, so the
 // compiler can wait for exactly the loads a row needs instead of all of them.
@@ -529,7 +516,7 @@ __device__ __forceinline__ NbRow normb_row_load(const GemmArgs& p, int row, int 
   }
   return in;
 }
-// The row's norm backward from its preloaded operands (normb_apply's arithmetic).
+// The row's norm backward from its preloaded operands.
 __device__ __forceinline__ void normb_row_apply(const GemmArgs& p, float4 gg, int row, int col, const NbRow& in,
                                                 const float4& g, float4& dw) {
   const bool on = row < p.M;
@@ -555,67 +542,6 @@ __device__ __forceinline__ void normb_row_apply(const GemmArgs& p, float4 gg, in
   o.y += in.add.y + in.addl.y;
   o.z += in.add.z + in.addl.z;
   o.w += in.add.w + in.addl.w;
-  *reinterpret_cast<float4*>(p.nb_dx + (long long)row * p.N + col) = o;
-}
-
-template <bool PRE>
-__device__ __forceinline__ void normb_apply(const GemmArgs& p, float4 gg, int row, int col, const NbIn& in,
-                                            const float4& g, float4& dw) {
-  const bool on = row < p.M;
-  if constexpr (PRE) {  // the addend sum_h P[row][h] U[sample][h] (E_NBPRE), before anything else
-    if (on) {
-      const float4 w = *reinterpret_cast<const float4*>(p.nb_pre_p + (long long)row * 4);
-      const float* u = p.nb_pre_u + (long long)(row / p.nb_seq) * 4 * p.N + col;
-      const float wh[4] = {w.x, w.y, w.z, w.w};
-      float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const float4 uh = *reinterpret_cast<const float4*>(u + t * p.N);
-        a = make_float4(fmaf(wh[t], uh.x, a.x), fmaf(wh[t], uh.y, a.y), fmaf(wh[t], uh.z, a.z), fmaf(wh[t], uh.w, a.w));
-      }
-      gg.x += a.x;
-      gg.y += a.y;
-      gg.z += a.z;
-      gg.w += a.w;
-    }
-  }
-  // the addend row, issued first: its latency runs under the row reduction below
-  const float4 add = on && p.nb_add ? *reinterpret_cast<const float4*>(p.nb_add + (long long)row * p.N + col)
-                                    : make_float4(0.f, 0.f, 0.f, 0.f);
-  const bool last = (p.nb_add_last || p.nb_dy_last) && on &&
-                    row % p.nb_seq == last_row(p.nb_lens, row / p.nb_seq, p.nb_seq);
-  if (last && p.nb_dy_last) {
-    const float4 a = *reinterpret_cast<const float4*>(p.nb_dy_last + (long long)(row / p.nb_seq) * p.N + col);
-    gg.x += a.x;
-    gg.y += a.y;
-    gg.z += a.z;
-    gg.w += a.w;
-  }
-  if (!on) gg = make_float4(0.f, 0.f, 0.f, 0.f);
-  const float r = in.r;
-  const float4 xh = make_float4(in.x.x * r, in.x.y * r, in.x.z * r, in.x.w * r);
-  float dot = gg.x * g.x * xh.x + gg.y * g.y * xh.y + gg.z * g.z * xh.z + gg.w * g.w * xh.w;
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
-  const float md = dot * (1.0f / (float)p.N);
-  dw.x += gg.x * xh.x;
-  dw.y += gg.y * xh.y;
-  dw.z += gg.z * xh.z;
-  dw.w += gg.w * xh.w;
-  if (!on) return;
-  float4 o = make_float4(r * (gg.x * g.x - xh.x * md), r * (gg.y * g.y - xh.y * md), r * (gg.z * g.z - xh.z * md),
-                         r * (gg.w * g.w - xh.w * md));
-  o.x += add.x;
-  o.y += add.y;
-  o.z += add.z;
-  o.w += add.w;
-  if (last && p.nb_add_last) {
-    const float4 a = *reinterpret_cast<const float4*>(p.nb_add_last + (long long)(row / p.nb_seq) * p.N + col);
-    o.x += a.x;
-    o.y += a.y;
-    o.z += a.z;
-    o.w += a.w;
-  }
   *reinterpret_cast<float4*>(p.nb_dx + (long long)row * p.N + col) = o;
 }
 
@@ -858,7 +784,7 @@ __device__ __forceinline__ void stage_acc(float* T, const floatx16 (&acc)[MT][2]
 // incrementally (no division per row).
 // E_NBPRE on 64-row tiles: the four-term addend sum_h P[row][h] U[row / seq][h] added to the
 // thread's own staged rows of T (the rows and columns normb_rows then reads), four rows' P and U
-// loads in flight at once; normb_apply adds it to the product in the same order.
+// loads in flight at once.
 __device__ __forceinline__ void normb_pre_rows(const GemmArgs& p, float* T, int cg, int col, int r0) {
   constexpr int RT = T_ROWS / 8;
 #pragma unroll
@@ -1720,12 +1646,10 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
   const bool aligned = ((p.ldc & 3) == 0) && (((E & E_RESID) == 0) || (p.ldr & 3) == 0) &&
                        (((E & (E_GELU | E_RELU | E_DGELU | E_DRELU)) == 0) || (p.ldaux & 3) == 0) &&
                        ((reinterpret_cast<uintptr_t>(C) & 15) == 0);
-  // E_NORMB on 64-row tiles: the whole tile is staged at once, so no accumulator is live in the
-  // epilogue, and each thread keeps the x, rstd and addend rows of a few rows in flight ahead of
-  // the row it finishes (normb_rows). (On 128-row tiles the second half's accumulators are live
-  // through the first half's epilogue, which leaves registers for x one row ahead; there the
-  // epilogue phase of the lockstep grid runs at the bandwidth of its mixed reads and writes, and
-  // deeper prefetching of the second half measured the same.)
+  // E_NORMB: each thread keeps the x, rstd and addend rows of a few rows in flight ahead of the row
+  // it finishes (normb_rows). On 64-row tiles the whole tile is staged at once; on 128-row tiles
+  // each half, with the other half's accumulators live (one row ahead, as before the split
+  // products left registers for more, an epilogue took 37 k cycles of a 100 k cycle tile at K = 512).
   constexpr bool NB_PIPE = (E & E_NORMB) != 0 && MT == 1;
   if constexpr (NB_PIPE) {
     constexpr bool LAST = (E & E_NBLAST) != 0;
@@ -1771,29 +1695,10 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     } else if constexpr ((E & E_NORMB) != 0) {
       const float4 g = *reinterpret_cast<const float4*>(p.nb_gain + col);
       const int rbase = m0 + half * T_ROWS + (threadIdx.x >> 5);
-      // the next row's x and rstd load under this row's work; with E_NBPRE, after the row (its
-      // last-row terms leave no registers for them ahead: 16 bytes a lane spilled, 80.6 against
-      // 79.3 us at C4), and the addend's P and U loaded in the row's own step unless the products
-      // already added it (82.3 us when they did not)
-      const bool pre = (E & E_NBPRE) != 0 && !pre_folded;
-      NbIn cur = normb_load(p, rbase, col);
-#pragma unroll 1
-      for (int i = 0; i < T_ROWS / 8; ++i) {
-        const int lr = (threadIdx.x >> 5) + 8 * i;
-        NbIn nxt = cur;
-        if ((E & E_NBPRE) == 0 && i + 1 < T_ROWS / 8) nxt = normb_load(p, rbase + 8 * (i + 1), col);
-        const float4 v = *reinterpret_cast<const float4*>(T + lr * T_S + cg);
-        if constexpr ((E & E_NBPRE) != 0) {
-          if (pre)
-            normb_apply<true>(p, v, rbase + 8 * i, col, cur, g, nbw);
-          else
-            normb_apply<false>(p, v, rbase + 8 * i, col, cur, g, nbw);
-        } else {
-          normb_apply<false>(p, v, rbase + 8 * i, col, cur, g, nbw);
-        }
-        if ((E & E_NBPRE) != 0 && i + 1 < T_ROWS / 8) nxt = normb_load(p, rbase + 8 * (i + 1), col);
-        cur = nxt;
-      }
+      if constexpr ((E & E_NBPRE) != 0)
+        if (!pre_folded) normb_pre_rows(p, T, cg, col, rbase);
+      constexpr bool LAST = (E & E_NBLAST) != 0;
+      normb_rows<LAST ? TALOS_NB_AHEAD_LAST : TALOS_NB_AHEAD, LAST>(p, T, cg, col, rbase, g, nbw);
     } else {
       // the row-dependent operands of four rows at a time (and the bias once) are loaded before
       // those rows' stores
