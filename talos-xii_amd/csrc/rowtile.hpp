@@ -168,6 +168,16 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// The largest over aligned groups of 8 lanes, in every lane of the group.
+__device__ __forceinline__ float group8_max(float v) {
+  auto dpp = [](float x, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xF, 0xF, false));
+  };
+  v = fmaxf(v, dpp(v, std::integral_constant<int, 0xB1>{}));
+  v = fmaxf(v, dpp(v, std::integral_constant<int, 0x4E>{}));
+  return fmaxf(v, dpp(v, std::integral_constant<int, 0x141>{}));
+}
+
 // y = x / sqrt(mean(x^2) + eps) * g over the 16 rows, 16 lanes per row (threads 0..255; the
 // rstd of each row optionally stored); the lane's gains are loaded by RowGain::load ahead of the
 // phase.
