@@ -523,6 +523,22 @@ __global__ __launch_bounds__(512) void attn_fwd_s64_wo_kernel(AttnArgs a, WoArgs
 // ---------------------------------------------------------------------------
 constexpr int kQTile = 128;  // queries per workgroup (4 waves x 32)
 
+// The (batch, head) pair and the tile of a workgroup. Under a causal mask a tile of all pairs comes
+// before the next tile, the one with the most blocks first (the last query tile, the first key tile):
+// side by side, two tiles a pair put every short one on the even XCDs and every long one on the odd
+// ones (24 x 200 tokens, 8 heads of 64, forward and backward: 177 -> 145 us). Without a mask the tiles
+// are equally long and stay side by side (the latent block of 64 x 256 tokens measured the
+// same either way, 1283 and 1289 us on two boxes).
+struct PairTile {
+  int pair, tile;
+};
+__device__ __forceinline__ PairTile pair_tile(const AttnArgs& a, int ntile, bool last_first) {
+  const int i = blockIdx.x;
+  if (!a.causal) return {i / ntile, i % ntile};
+  const int np = a.B * a.H, t = i / np;
+  return {i - t * np, last_first ? ntile - 1 - t : t};
+}
+
 // Element group g (4 consecutive floats) of a [32 rows, DM] block starting at row0: row 4g / DM,
 // column 4g % DM; rows >= nrows and columns >= dim read as 0.
 template <int DM>
@@ -587,7 +603,8 @@ attn_fwd_tiled_kernel(AttnArgs a) {
   __shared__ __align__(16) float Wr[4][32];
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, true);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int Sk = key_len(a, b);
@@ -870,7 +887,8 @@ attn_bwd_dq_tiled_kernel(AttnArgs a) {
   __shared__ __align__(16) float Vs[32 * PV];
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, true);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int Sk = key_len(a, b);
@@ -1013,7 +1031,8 @@ attn_bwd_dkv_tiled_kernel(AttnArgs a) {
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int t = threadIdx.x;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, false);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int kb = tile * 4 + wv;  // this wave's key block
@@ -1213,7 +1232,8 @@ attn_bwd_dq_ds_kernel(AttnArgs a) {
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int t = threadIdx.x;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, true);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int Sk = key_len(a, b);
@@ -1392,7 +1412,8 @@ attn_fwd_tiled_bf16_kernel(AttnArgs a) {
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int t = threadIdx.x;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, true);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int Sk = key_len(a, b);
@@ -1515,7 +1536,8 @@ attn_bwd_dkv_bf16_kernel(AttnArgs a) {
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int t = threadIdx.x;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, false);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int kb = tile * 4 + wv;
@@ -1674,7 +1696,8 @@ attn_bwd_dq_ds_bf16_kernel(AttnArgs a) {
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
   const int t = threadIdx.x;
   const int ntile = (a.S + kQTile - 1) / kQTile;
-  const int pair = blockIdx.x / ntile, tile = blockIdx.x % ntile;
+  const PairTile pt = pair_tile(a, ntile, true);
+  const int pair = pt.pair, tile = pt.tile;
   const int b = pair / a.H, hd = pair % a.H;
   const long long tok0 = (long long)b * a.S;
   const int Sk = key_len(a, b);
