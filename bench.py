@@ -32,6 +32,7 @@ METRIC = "PPO policy fwd+bwd samples/sec (d128 block, 1 GPU); % MFMA/HBM rooflin
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 PEAK_BF16_MFMA_TFLOPS = 2516.6
+PEAK_SPLIT_TFLOPS = round(PEAK_BF16_MFMA_TFLOPS / 6, 1)  # the fp32 GEMMs: six bf16 products each
 
 
 def ppo_cfg(B, S):
@@ -72,11 +73,12 @@ def runs_on_bf16_mfma(name):
 def roofline_of(name, n, flops, bytes_, ms, peak_tflops=None):
     """The roofline of a kernel symbol from its launches: matrix-core bound when its arithmetic
     intensity (algorithmic flops per algorithmic HBM byte) is above the ridge point of the MFMA
-    peak it runs on (fp32 157.3 TFLOP/s, or bf16 2.5 PFLOP/s for the bf16-in GEMMs), HBM-bound
-    below it. achieved = algorithmic work per launch / average launch time."""
+    peak it runs on (fp32 157.3 TFLOP/s, bf16 2.5 PFLOP/s for the bf16-in GEMMs, a sixth of that
+    for the fp32 GEMMs, whose products are six bf16 ones), HBM-bound below it. achieved = algorithmic work per launch / average launch time."""
     avg_ms = ms / n
     if peak_tflops is None:
-        peak_tflops = PEAK_BF16_MFMA_TFLOPS if runs_on_bf16_mfma(name) else PEAK_FP32_MFMA_TFLOPS
+        peak_tflops = (PEAK_BF16_MFMA_TFLOPS if runs_on_bf16_mfma(name) else
+                       PEAK_SPLIT_TFLOPS if name.startswith("gemm_") else PEAK_FP32_MFMA_TFLOPS)
     ridge = peak_tflops * 1e12 / (PEAK_HBM_GBS * 1e9)
     if flops > 0 and (bytes_ <= 0 or flops / bytes_ >= ridge):
         achieved = flops / n / (avg_ms * 1e-3) / 1e12
