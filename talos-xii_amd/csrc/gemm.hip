@@ -1,11 +1,13 @@
-// gemm.hip -- fp32 GEMM on CDNA4 matrix cores (v_mfma_f32_32x32x2_f32) for gfx950.
+// gemm.hip -- fp32 and bf16-in GEMM on the CDNA4 matrix cores for gfx950.
 //
 // Replaces the row-accumulation matmul of the reference and its backward
 // (src/autograd.rs:200-354): forward C = A.B, dA += dC.B^T, dB += A^T.dC, plus the batched
 // Q.K^T / P.V products of attention (src/transformer.rs:877-1050).
 //
 // Tiling: a 256-thread workgroup owns a 128x128 tile of C; each of its four waves owns a
-// 64x64 quarter as 2x2 MFMA 32x32 accumulators (64 accumulator registers per lane). K advances
+// 64x64 quarter as 2x2 MFMA 32x32 accumulators (64 accumulator registers per lane).
+// fp32 products are formed from bf16 splits (below, "fp32 products on the bf16 matrix cores"); the
+// chain described here forms a tile again where a sum of the split products is not finite. K advances
 // in chunks of 32 staged through LDS; the next chunk is fetched into registers while the matrix
 // cores work on the current one. Each operand panel keeps the layout the operand has in memory:
 // k-contiguous operands (A plain, B transposed) as rows of 32 k values (pitch 36), read by the
@@ -37,12 +39,9 @@ constexpr int KP = 36;
 constexpr int PANEL = (BK * LDS_S > 128 * KP) ? BK * LDS_S : 128 * KP;  // floats per panel
 constexpr int NT = 256;
 // Tuning knobs (compile-time): TALOS_GEMM_DBUF = 1 double-buffers the LDS panels (one barrier per
-// K chunk); TALOS_GEMM_WAVES = minimum waves per SIMD the register allocation must allow.
+// K chunk).
 #ifndef TALOS_GEMM_DBUF
 #define TALOS_GEMM_DBUF 0
-#endif
-#ifndef TALOS_GEMM_WAVES
-#define TALOS_GEMM_WAVES 4
 #endif
 // Split-K sizing: target workgroups per CU and the minimum K per split (512: at 32768 tokens the
 // weight gradients take 64 splits instead of 128, C3 0.614-0.620 -> 0.608-0.609 ms; 768 and 1024
