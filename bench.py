@@ -159,7 +159,7 @@ def cpu_baseline_c5(seconds=6.0):
 def cpu_baseline(cfg_t, seconds_budget=20.0):
     """The f64 oracle on this host: reference-faithful per-sample batch-1 graphs (the backbone run
     for the actor and again for the critic, src/ppo.rs:691-757) on a bounded sample, plus the
-    batched restatement. Threads: this host's cores, at most 16 (a GPU box's CPU share)."""
+    batched restatement. Threads: this host's cores, at most 16."""
     import pyoracle  # prebuilt by __graft_entry__.build(); never compiled from a GPU process
     threads = max(1, min(16, len(os.sched_getaffinity(0))))
     pyoracle.set_threads(threads)
