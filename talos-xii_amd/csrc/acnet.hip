@@ -291,8 +291,10 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < D / 16; ++c) ss = fmaf(h[c][r], h[c][r], ss);
-        const float rs = 1.0f / sqrtf(group_sum<16>(ss) / (float)D + k.eps);
+        // rows past nt are zeros: rstd 0 there, as 1 / sqrt(0 + eps) is infinite for eps = 0 and the
+        // products over whole tiles would take 0 * inf into every gradient of the token weights
         const int t = 16 * w + 4 * kq + r;
+        const float rs0 = 1.0f / sqrtf(group_sum<16>(ss) / (float)D + k.eps), rs = t < nt ? rs0 : 0.f;
         if (i == 0) sm.rs[t] = rs;
 #pragma unroll
         for (int c = 0; c < D / 16; ++c) sm.X[t * LX + 16 * c + i] = h[c][r] * rs * sm.g1[16 * c + i];

@@ -90,6 +90,21 @@ def test_one_kernel_matches_separate_products(monkeypatch, n, batch, S, ragged, 
     compare(got, ref, A)
 
 
+@pytest.mark.parametrize("n,S", [(8, 15), (1, 15), (9, 17), (5, 16)])
+def test_eps_zero(monkeypatch, n, S):
+    """Token tiles that are not full (a group's tokens no multiple of 16, a last group of one sample) hold
+    zero rows, whose 1 / sqrt(0 + eps) must not reach the gradients."""
+    rng = np.random.default_rng(31 * n + S)
+    a = list(net_args(n, S, th.ACT_GELU))
+    assert a[11] == 1e-5
+    a[11] = 0.0
+    cfg = th.PpoCfg(*a)
+    p = f32(ppo_params(rng, cfg)).astype(np.float32)
+    got, ref = both(monkeypatch, cfg, n, p, *inputs(rng, n, S, 5, False))
+    assert np.all(np.isfinite(got[1]))
+    compare(got, ref, 5)
+
+
 def test_out_of_range_action(monkeypatch):
     """NaN loss, and no gradient from that sample, as on the other path."""
     rng = np.random.default_rng(77)
