@@ -960,7 +960,18 @@ int group_size(const talos_ppo_cfg& c, int n, int num_cu) {
   return std::max(1, std::min(most, n / std::max(1, num_cu / 4)));
 }
 
-KArgs make_args(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, unsigned* grid) {
+// Workgroups (and partial rows) of a minibatch: one a CU, more where the fp32 accumulators of a
+// workgroup would then run over more than 512 tokens or 256 samples (the runs of the separate
+// products' split weight gradients and row chunks, whose partials are added in f64 as these are).
+// A later round of workgroups takes what the earlier one left: nothing else changes, and a row
+// more is 178 KB written for at least 170 us of work.
+unsigned minibatch_grid(int ngroups, int group_tokens, int num_cu) {
+  const int run = std::max(1, std::min(256 / GS, 512 / group_tokens));
+  const long long rounds = ceil_div((size_t)ngroups, (size_t)run * num_cu);
+  return (unsigned)std::min<long long>(ngroups, rounds * num_cu);
+}
+
+KArgs make_args(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, bool backward, unsigned* grid) {
   KArgs k{};
   k.B = a.n;
   k.S = c.seq;
@@ -976,7 +987,7 @@ KArgs make_args(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, unsigned
   k.vec = (reinterpret_cast<uintptr_t>(a.states) & 15) == 0;
   k.pitch = param_pitch(c.n_actions);
   k.c = a;
-  *grid = (unsigned)std::min(k.ngroups, num_cu);
+  *grid = backward ? minibatch_grid(k.ngroups, k.G * k.S, num_cu) : (unsigned)std::min(k.ngroups, num_cu);
   return k;
 }
 
@@ -994,12 +1005,15 @@ bool acnet_supported(const talos_ppo_cfg& c) {
 }
 
 size_t acnet_ws_bytes(const talos_ppo_cfg& c, int num_cu) {
-  return (size_t)num_cu * (kStats * sizeof(double) + param_pitch(c.n_actions) * sizeof(float));
+  // (a call of fewer samples has fewer rows: its groups are whole ones, or no more than CUs)
+  const int most = std::min(GS, T / c.seq);
+  const size_t rows = std::max((unsigned)num_cu, minibatch_grid((int)ceil_div((size_t)c.batch, most), most * c.seq, num_cu));
+  return rows * (kStats * sizeof(double) + param_pitch(c.n_actions) * sizeof(float));
 }
 
 int acnet_forward_launch(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, hipStream_t s) {
   unsigned grid;
-  const KArgs k = make_args(c, num_cu, a, &grid);
+  const KArgs k = make_args(c, num_cu, a, false, &grid);
   ProfScope ps(s, "acnet_kernel<false>", flops_of(c, a.n), 4.0 * a.n * (c.seq * IN + c.n_actions + 1.0));
   hipLaunchKernelGGL(acnet_kernel<false>, dim3(grid), dim3(NTHR), 0, s, k);
   return launch_status("acnet_kernel");
@@ -1007,9 +1021,9 @@ int acnet_forward_launch(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a,
 
 int acnet_minibatch_launch(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, hipStream_t s) {
   unsigned grid;
-  KArgs k = make_args(c, num_cu, a, &grid);
+  KArgs k = make_args(c, num_cu, a, true, &grid);
   k.stat_part = a.ws;
-  k.part = reinterpret_cast<float*>(a.ws + (size_t)num_cu * kStats);
+  k.part = reinterpret_cast<float*>(a.ws + (size_t)grid * kStats);
   const int np = oWA + D * c.n_actions + c.n_actions + D + 1;
   {
     ProfScope ps(s, "acnet_kernel<true>", 3.0 * flops_of(c, a.n), 4.0 * a.n * c.seq * IN + 4.0 * grid * k.pitch);

@@ -105,6 +105,44 @@ def test_eps_zero(monkeypatch, n, S):
     compare(got, ref, 5)
 
 
+# The flat tensors in order
+TENSORS = "we be g1 wdkv wuk wuv wq wkr wqr wo g2 w1 b1 w2 b2 gf wout bout wa ba wc bc".split()
+
+
+def test_small_terms_after_a_large_one():
+    """65536 equal samples, the first with advantage and value error 1, the others with 2^-26: every
+    gradient is the one sample's times 1 + 65535 * 2^-26 (all scales are powers of two, so each sample's own
+    terms are exactly scaled copies). An fp32 sum that starts with the first sample keeps none of the
+    terms after it, and loses 2^-26 a sample: a workgroup's run of at most 32 samples (512 tokens) 31 * 2^-26,
+    and the final rounding and the sums over tokens a few 2^-24, below 2^-20 together. (A run over all of a CU's
+    256 samples loses 3.8e-6.) Elementwise, relative to the tensor's largest value."""
+    n, S = 65536, 16
+    a = list(net_args(n, S, th.ACT_GELU))
+    a[15] = 0.0  # no entropy term: its gradient would not scale
+    rng = np.random.default_rng(5)
+    p = f32(ppo_params(rng, th.PpoCfg(*a))).astype(np.float32)
+    p[-65:] = 0.0  # value 0 exactly
+    small = np.float32(2.0**-26)
+    one = f32(gacha_states(rng, 1, S)).astype(np.float32)
+
+    def grads(B, count):
+        a[0] = B
+        scale = np.full(count, small, np.float32)
+        scale[0] = 1.0
+        # (a negative advantage and a ratio above 1 + clip: never clipped)
+        return run(th.PpoCfg(*a), count, p, np.tile(one, (count, 1, 1)), None, np.full(count, 2, np.int32), -scale, -scale,
+                   np.full(count, -6.0, np.float32))[1]
+
+    ref = grads(1, 1) * (1.0 + (n - 1) * float(small)) / n
+    got, o = grads(n, n), 0
+    for name, size in zip(TENSORS, tensor_sizes(5)):
+        g, r = got[o:o + size], ref[o:o + size]
+        o += size
+        assert np.abs(r).max() > 0, name
+        err = np.abs(g - r).max() / np.abs(r).max()
+        assert err <= 2.0**-20, (name, err)
+
+
 def test_out_of_range_action(monkeypatch):
     """NaN loss, and no gradient from that sample, as on the other path."""
     rng = np.random.default_rng(77)
