@@ -14,13 +14,14 @@
 // written to memory. The products run on v_mfma_f32_16x16x4f32: token products with 16 tokens as
 // the tile rows (a wave a tile), sample products with the 8 samples as half a tile, the weight
 // gradients with tokens or samples as k into accumulators that stay in registers over all of the
-// workgroup's samples. At the end a workgroup writes its parameter gradients once as a partial
+// workgroup's samples (at most 512 tokens or 256 samples: minibatch_grid); the gains' and the heads'
+// gradients add in f64. At the end a workgroup writes its parameter gradients once as a partial
 // row; acnet_reduce_kernel adds the rows in a fixed order in f64.
 //
 // Bound by the latency of its 28 dependent phases (LDS round trips and barriers, one workgroup per
 // CU: 160 KB of LDS; about 95 k cycles a group of 8 samples x 16 tokens, 25 k of them in the four
 // token-product phases, which run at about half of the fp32 matrix rate), then by the partial rows
-// (178 KB a workgroup). One MI355X, minibatch forward + backward: 4096 x 16 tokens 849 -> 87 us,
+// (181 KB a workgroup). One MI355X, minibatch forward + backward: 4096 x 16 tokens 849 -> 87 us,
 // 256 ragged samples of up to 16 tokens 411 -> 39 us.
 #include "acnet.hpp"
 
@@ -84,11 +85,13 @@ struct KArgs {
   int B, S, G, ngroups, A, relu;
   float eps, scale, clip_eps, cv, ce;
   int vec;  // 16-byte states rows
-  int pitch;  // floats of a partial row
+  int pitch, dpitch;  // floats and doubles of a partial row
   AcNetCall c;
-  float* part;
+  float* part;        // [workgroups][pitch], at the parameters' offsets
+  double* dpart;      // [workgroups][dpitch]: dg1 | dg2 | dgf | the heads
   double* stat_part;  // [workgroups][kStats]
 };
+typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 // the lane's weights of a 16-column tile, column n: k = k0 + 16 g + 4 kq + u
 template <int K, bool TRANS>
@@ -208,8 +211,11 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
 
   // gradient accumulators (tile t of a matrix on wave t % 8 unless said otherwise)
   const rt_floatx4 z4 = {0.f, 0.f, 0.f, 0.f};
-  rt_floatx4 gK[3], gQ[4], gUK = z4, gUV = z4, gE = z4, gOut[2], gW2[4], gW1[4], gWo[2], gH = z4;
-  float agf = 0.f, ag2 = 0.f, about = 0.f, ab2 = 0.f, ab1 = 0.f, abh = 0.f;
+  rt_floatx4 gK[3], gQ[4], gUK = z4, gUV = z4, gE = z4, gOut[2], gW2[4], gW1[4], gWo[2];
+  float about = 0.f, ab2 = 0.f, ab1 = 0.f;
+  // the gains' and the heads' gradients add in f64, as their kernels in the separate products do
+  doublex4 gH = {0.0, 0.0, 0.0, 0.0};
+  double ag1 = 0.0, agf = 0.0, ag2 = 0.0, abh = 0.0;
   if constexpr (BWD) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) gK[q] = z4;
@@ -560,7 +566,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         sm.po[w * LR + lane] = pr;
         const float dzv = lane < MAXA ? dzf : lane == MAXA ? dvf : 0.f;
         if (lane < 16) sm.dz[w * 16 + lane] = dzv;
-        abh += dzv;
+        abh += (double)dzv;
         about += g;
         sm.gpo[w * LR + lane] = g;
       }
@@ -578,7 +584,12 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
           const int t = w + 8 * q;
           mm_grad(gOut[q], kq, sm.ln + 16 * (t >> 2) + i, LR, sm.gpo + 16 * (t & 3) + i, LR);
         }
-        if (w < 4) mm_grad(gH, kq, sm.po + 16 * w + i, LR, sm.dz + i, 16);
+        if (w < 4) {
+#pragma unroll
+          for (int s = 0; s < GS / 4; ++s)
+            gH = __builtin_amdgcn_mfma_f64_16x16x4f64((double)sm.po[(4 * s + kq) * LR + 16 * w + i],
+                                                      (double)sm.dz[(4 * s + kq) * 16 + i], gH, 0, 0, 0);
+        }
       }
       lds_barrier();
       // ---- the final norm's backward
@@ -587,7 +598,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         const float xh = sm.last[w * LR + lane] * r;
         const float md = wave_total(dy * gf * xh) * (1.0f / (float)D);
         const float g = r * (dy * gf - xh * md);
-        agf += dy * xh;
+        agf += (double)(dy * xh);
         ab2 += g;
         sm.last[w * LR + lane] = g;
       }
@@ -625,7 +636,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         const float dy = sm.po[w * LR + lane] + sm.xl[w * LR + lane], r = sm.r2[w];
         const float xh = sm.h2[w * LR + lane] * r;
         const float md = wave_total(dy * g2 * xh) * (1.0f / (float)D);
-        ag2 += dy * xh;
+        ag2 += (double)(dy * xh);
         sm.last[w * LR + lane] += r * (dy * g2 - xh * md);
       }
       float wuvT[4];
@@ -813,16 +824,19 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
         }
       }
       lds_barrier();
-      // ---- dWe and dbe (the states' column of ones) as rows 0 .. 8 of a tile, dg1 as row 9; tokens
-      // of alternate tiles on the wave pairs
-      for (int b = kh; b < ntile; b += 2)
+      // ---- dWe and dbe (the states' column of ones) as rows 0 .. 8 of a tile, dg1 as the sums over
+      // each tile's 16 tokens (every row of g1t) added in f64; tokens of alternate tiles on the wave pairs
+      for (int b = kh; b < ntile; b += 2) {
+        rt_floatx4 g1t = z4;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const int tok = 16 * b + 4 * kq + s;
           const float x = i <= IN ? sm.St[tok * LS + i] : 0.f;
           gE = __builtin_amdgcn_mfma_f32_16x16x4f32(x, sm.X[tok * LX + n4], gE, 0, 0, 0);
-          gE = __builtin_amdgcn_mfma_f32_16x16x4f32(i == IN + 1 ? 1.f : 0.f, sm.C[tok * LC + n4], gE, 0, 0, 0);
+          g1t = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, sm.C[tok * LC + n4], g1t, 0, 0, 0);
         }
+        ag1 += (double)g1t[0];
+      }
     }
     lds_barrier();  // the next group's phases write what these read
   }
@@ -830,6 +844,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     // ---- this workgroup's partial row
     const int n4 = (w & 3) * 16 + i, kh = w >> 2, hd2 = w >> 1, hf = w & 1;
     float* G = k.part + (long long)blockIdx.x * k.pitch;
+    double* GD = k.dpart + (long long)blockIdx.x * k.dpitch;
     auto tile = [&](const rt_floatx4& v, int off, int ld, int m, int n) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) G[off + (16 * m + 4 * kq + r) * ld + 16 * n + i] = v[r];
@@ -859,39 +874,42 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     }
     ab1 += __shfl_xor(ab1, 16, 64);  // (lane quarters 2 and 3 hold zeros)
     if (kq == 0) G[oB1 + 16 * w + i] = ab1;
-    if (w < 4) {
+    if (w < 4) {  // (register r of an f64 tile is row 4 r + kq)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int f = 16 * w + 4 * kq + r;
-        if (i < A) G[oWA + f * A + i] = gH[r];
-        if (i == MAXA) G[oWA + D * A + A + f] = gH[r];
+        const int f = 16 * w + 4 * r + kq;
+        if (i < A) GD[3 * D + f * A + i] = gH[r];
+        if (i == MAXA) GD[3 * D + D * A + A + f] = gH[r];
       }
     }
-    // sums over the waves (samples) through LDS, in f64, and the two halves of the embedding's tile
-    float* R = sm.C;  // [8 waves][5][64]
-    float* E = sm.X;  // [2][16][64]
+    // sums over the waves (samples) through LDS, in f64, the two halves of the embedding's tile and of dg1
+    double* R = reinterpret_cast<double*>(sm.C);           // [8 waves][5][64]
+    float* E = sm.X;                                       // [2][16][64]
+    double* E1 = reinterpret_cast<double*>(sm.X + 2 * 1024);  // [2][64]
     {
-      float* r = R + w * 320 + lane;
+      double* r = R + w * 320 + lane;
       r[0] = agf;
       r[64] = ag2;
-      r[128] = about;
-      r[192] = ab2;
-      r[256] = abh;
+      r[128] = abh;
+      r[192] = (double)about;
+      r[256] = (double)ab2;
 #pragma unroll
       for (int q = 0; q < 4; ++q) E[kh * 1024 + (4 * kq + q) * 64 + n4] = gE[q];
+      if (kq == 0) E1[kh * 64 + n4] = ag1;
     }
     lds_barrier();
     if (tid < 320) {
       const int row = tid >> 6;
       double s = 0.0;
 #pragma unroll
-      for (int q = 0; q < NWV; ++q) s += (double)R[q * 320 + tid];
-      const float v = (float)s;
-      if (row < 4) G[(row == 0 ? oGF : row == 1 ? oG2 : row == 2 ? oBOUT : oB2) + lane] = v;
-      else if (lane < A) G[oWA + D * A + lane] = v;
-      else if (lane == MAXA) G[oWA + D * A + A + D] = v;
+      for (int q = 0; q < NWV; ++q) s += R[q * 320 + tid];
+      if (row < 2) GD[(row == 0 ? 2 * D : D) + lane] = s;
+      else if (row > 2) G[(row == 3 ? oBOUT : oB2) + lane] = (float)s;
+      else if (lane < A) GD[3 * D + D * A + lane] = s;
+      else if (lane == MAXA) GD[3 * D + D * A + A + D] = s;
     }
-    for (int e = tid; e < (IN + 2) * D; e += NTHR) G[oWE + e] = E[e] + E[1024 + e];  // be and g1 follow we
+    if (tid < D) GD[tid] = E1[tid] + E1[D + tid];
+    for (int e = tid; e < (IN + 1) * D; e += NTHR) G[oWE + e] = E[e] + E[1024 + e];  // be follows we
     if (tid < kStats) {
       double s = 0.0;
 #pragma unroll
@@ -901,11 +919,28 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
   }
 }
 
-// dparams[e] = the workgroups' partial rows added in a fixed order in f64: 64 consecutive elements
-// a workgroup, wave w the rows w, w + 4, ... in four accumulators; the last workgroup adds the
-// loss statistics.
-__global__ __launch_bounds__(256) void acnet_reduce_kernel(int nwg, int nparams, int pitch, int B,
+// dparams[e] = the workgroups' partial rows (f64 for the gains and the heads, fp32 for the rest)
+// added in a fixed order in f64: 64 consecutive elements a workgroup, wave w the rows w, w + 4, ...
+// in four accumulators; the last workgroup adds the loss statistics.
+template <class V>
+__device__ __forceinline__ double column_sum(int nwg, int w, const V* __restrict__ q, long long pitch) {
+  const long long st = 4 * pitch;
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  int g = w;
+  q += w * pitch;
+  for (; g + 12 < nwg; g += 16, q += 4 * st) {
+    const V a = q[0], b = q[st], c = q[2 * st], d = q[3 * st];
+    s0 += (double)a;
+    s1 += (double)b;
+    s2 += (double)c;
+    s3 += (double)d;
+  }
+  for (; g < nwg; g += 4, q += st) s0 += (double)q[0];
+  return (s0 + s1) + (s2 + s3);
+}
+__global__ __launch_bounds__(256) void acnet_reduce_kernel(int nwg, int nparams, int pitch, int dpitch, int B,
                                                            const float* __restrict__ part,
+                                                           const double* __restrict__ dpart,
                                                            const double* __restrict__ stat_part,
                                                            float* __restrict__ dparams, float* __restrict__ loss,
                                                            double* __restrict__ stats, int stats_acc) {
@@ -928,27 +963,20 @@ __global__ __launch_bounds__(256) void acnet_reduce_kernel(int nwg, int nparams,
     }
     return;
   }
-  const int e = blockIdx.x * 64 + lane;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  if (e < nparams) {
-    const long long st = 4LL * pitch;
-    const float* q = part + (long long)w * pitch + e;
-    int g = w;
-    for (; g + 12 < nwg; g += 16, q += 4 * st) {
-      const float a = q[0], b = q[st], c = q[2 * st], d = q[3 * st];
-      s0 += (double)a;
-      s1 += (double)b;
-      s2 += (double)c;
-      s3 += (double)d;
-    }
-    for (; g < nwg; g += 4, q += st) s0 += (double)q[0];
-  }
-  red[w][lane] = (s0 + s1) + (s2 + s3);
+  // (the f64 sections start and end at multiples of 64)
+  const int e0 = blockIdx.x * 64, e = e0 + lane;
+  const int d0 = e0 == oG1 ? 0 : e0 == oG2 ? D : e0 == oGF ? 2 * D : e0 >= oWA ? 3 * D + e0 - oWA : -1;
+  double sum = 0.0;
+  if (e < nparams) sum = d0 < 0 ? column_sum(nwg, w, part + e, pitch) : column_sum(nwg, w, dpart + d0 + lane, dpitch);
+  red[w][lane] = sum;
   __syncthreads();
   if (w == 0 && e < nparams) dparams[e] = (float)((red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]));
 }
 
-int param_pitch(int A) { return (oWA + D * A + A + D + 1 + 63) / 64 * 64; }
+static_assert(oG1 % 64 == 0 && oG2 % 64 == 0 && oGF % 64 == 0 && oWA % 64 == 0 && D == 64, "acnet_reduce_kernel's sections");
+constexpr int kPitch = oWA;  // a row's floats: the parameters before the heads
+int dpart_pitch(int A) { return 3 * D + D * A + A + D + 1; }
+size_t row_bytes(int A) { return (kStats + dpart_pitch(A)) * sizeof(double) + kPitch * sizeof(float); }
 
 // Samples a workgroup takes at a time: as many as its 128 tokens hold (at most 8), fewer where the
 // batch would then leave more than three quarters of the CUs without work. (Not all the way down
@@ -964,7 +992,7 @@ int group_size(const talos_ppo_cfg& c, int n, int num_cu) {
 // workgroup would then run over more than 512 tokens or 256 samples (the runs of the separate
 // products' split weight gradients and row chunks, whose partials are added in f64 as these are).
 // A later round of workgroups takes what the earlier one left: nothing else changes, and a row
-// more is 178 KB written for at least 170 us of work.
+// more is 181 KB written for at least 170 us of work.
 unsigned minibatch_grid(int ngroups, int group_tokens, int num_cu) {
   const int run = std::max(1, std::min(256 / GS, 512 / group_tokens));
   const long long rounds = ceil_div((size_t)ngroups, (size_t)run * num_cu);
@@ -985,7 +1013,8 @@ KArgs make_args(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, bool bac
   k.cv = c.value_coef;
   k.ce = c.entropy_coef;
   k.vec = (reinterpret_cast<uintptr_t>(a.states) & 15) == 0;
-  k.pitch = param_pitch(c.n_actions);
+  k.pitch = kPitch;
+  k.dpitch = dpart_pitch(c.n_actions);
   k.c = a;
   *grid = backward ? minibatch_grid(k.ngroups, k.G * k.S, num_cu) : (unsigned)std::min(k.ngroups, num_cu);
   return k;
@@ -1008,7 +1037,7 @@ size_t acnet_ws_bytes(const talos_ppo_cfg& c, int num_cu) {
   // (a call of fewer samples has fewer rows: its groups are whole ones, or no more than CUs)
   const int most = std::min(GS, T / c.seq);
   const size_t rows = std::max((unsigned)num_cu, minibatch_grid((int)ceil_div((size_t)c.batch, most), most * c.seq, num_cu));
-  return rows * (kStats * sizeof(double) + param_pitch(c.n_actions) * sizeof(float));
+  return rows * row_bytes(c.n_actions);
 }
 
 int acnet_forward_launch(const talos_ppo_cfg& c, int num_cu, const AcNetCall& a, hipStream_t s) {
@@ -1023,16 +1052,17 @@ int acnet_minibatch_launch(const talos_ppo_cfg& c, int num_cu, const AcNetCall& 
   unsigned grid;
   KArgs k = make_args(c, num_cu, a, true, &grid);
   k.stat_part = a.ws;
-  k.part = reinterpret_cast<float*>(a.ws + (size_t)grid * kStats);
+  k.dpart = k.stat_part + (size_t)grid * kStats;
+  k.part = reinterpret_cast<float*>(k.dpart + (size_t)grid * k.dpitch);
   const int np = oWA + D * c.n_actions + c.n_actions + D + 1;
   {
-    ProfScope ps(s, "acnet_kernel<true>", 3.0 * flops_of(c, a.n), 4.0 * a.n * c.seq * IN + 4.0 * grid * k.pitch);
+    ProfScope ps(s, "acnet_kernel<true>", 3.0 * flops_of(c, a.n), 4.0 * a.n * c.seq * IN + (double)grid * row_bytes(c.n_actions));
     hipLaunchKernelGGL(acnet_kernel<true>, dim3(grid), dim3(NTHR), 0, s, k);
     if (int rc = launch_status("acnet_kernel")) return rc;
   }
-  ProfScope ps(s, "acnet_reduce_kernel", 0.0, 4.0 * (grid + 1.0) * np);
+  ProfScope ps(s, "acnet_reduce_kernel", 0.0, (double)grid * row_bytes(c.n_actions) + 4.0 * np);
   hipLaunchKernelGGL(acnet_reduce_kernel, dim3(ceil_div((size_t)np, 64) + 1), dim3(256), 0, s, (int)grid, np, k.pitch,
-                     a.n, k.part, k.stat_part, a.dparams, a.loss, a.stats, a.stats_acc);
+                     k.dpitch, a.n, k.part, k.dpart, k.stat_part, a.dparams, a.loss, a.stats, a.stats_acc);
   return launch_status("acnet_reduce_kernel");
 }
 

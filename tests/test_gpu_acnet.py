@@ -105,8 +105,9 @@ def test_eps_zero(monkeypatch, n, S):
     compare(got, ref, 5)
 
 
-# The flat tensors in order
+# The flat tensors in order, and those whose terms add in f64 over all samples
 TENSORS = "we be g1 wdkv wuk wuv wq wkr wqr wo g2 w1 b1 w2 b2 gf wout bout wa ba wc bc".split()
+F64_SUMS = "g1 g2 gf wa ba wc bc".split()
 
 
 def test_small_terms_after_a_large_one():
@@ -115,7 +116,8 @@ def test_small_terms_after_a_large_one():
     terms are exactly scaled copies). An fp32 sum that starts with the first sample keeps none of the
     terms after it, and loses 2^-26 a sample: a workgroup's run of at most 32 samples (512 tokens) 31 * 2^-26,
     and the final rounding and the sums over tokens a few 2^-24, below 2^-20 together. (A run over all of a CU's
-    256 samples loses 3.8e-6.) Elementwise, relative to the tensor's largest value."""
+    256 samples loses 3.8e-6.) The sums that are f64 throughout keep only the 2^-24 or so of their
+    own terms and of the result's rounding: 2^-23. Elementwise, relative to the tensor's largest value."""
     n, S = 65536, 16
     a = list(net_args(n, S, th.ACT_GELU))
     a[15] = 0.0  # no entropy term: its gradient would not scale
@@ -140,7 +142,7 @@ def test_small_terms_after_a_large_one():
         o += size
         assert np.abs(r).max() > 0, name
         err = np.abs(g - r).max() / np.abs(r).max()
-        assert err <= 2.0**-20, (name, err)
+        assert err <= (2.0**-23 if name in F64_SUMS else 2.0**-20), (name, err)
 
 
 def test_out_of_range_action(monkeypatch):
