@@ -993,8 +993,8 @@ __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb,
 // instead of 64: the error against f64 is 0.32x (K = 128) to 0.34x (K = 2048) of the fp32 chain's
 // (normal operands; 2.0e-7 -> 6.5e-8 and 8.1e-7 -> 2.8e-7 of the result's norm).
 // Values past the largest bf16 (3.39e38) and infinities have no such split: a tile whose sums are
-// not all finite is formed again by the fp32 chain. Below 2^-110 the third piece underflows: such a
-// value keeps an absolute accuracy of 2^-134.
+// not all finite is formed again by the fp32 chain. So is a tile that meets a nonzero value below
+// 2^-110, whose last bits are below bf16's least subnormal, 2^-133.
 //
 // Panels of SK = 16 k values a stage, two stages: chunk c is multiplied while chunk c + 1 (in
 // registers, loaded two chunks earlier) is split and stored to the other stage, one barrier a
@@ -1004,6 +1004,7 @@ __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb,
 // fragment reads fall on distinct banks.
 // ---------------------------------------------------------------------------
 constexpr int SK = 16;
+constexpr uint32_t kLeastSplit = 2u * (17u << 23) - 1u;  // 2^-110, as split3's least counts
 // the panel [ROWS x SK] of X at rows r0, k0, as fp32 (ROWS / 64 float4s a thread): KC: thread t
 // takes k 4 (t & 3) of rows t / 4 + 64 i; else columns 4 (t mod L) of k rows t / L + 8 i (L = ROWS / 4)
 template <bool KC, bool CHECK, int ROWS>
@@ -1026,9 +1027,21 @@ __device__ __forceinline__ void split_load(const float* __restrict__ X, long lon
     }
   }
 }
-// four values to their three bf16 pieces, packed
-__device__ __forceinline__ void split3(const float4& v, uint2 (&p)[3]) {
+// four values to their three bf16 pieces, packed. least: the least of the lane's nonzero magnitudes so
+// far, as twice the value's bits less one (a zero wraps to the largest). Six instructions beside the
+// split's 22, written out: left to the compiler they were hoisted over the products, 80 -> 108
+// registers on the 64 x 64 tiles (700 x 21 tokens, minibatch: 549 us without the check, 560 with it, 587 hoisted)
+__device__ __forceinline__ void split3(const float4& v, uint2 (&p)[3], uint32_t& least) {
   float r[4] = {v.x, v.y, v.z, v.w};
+  uint32_t t0, t1;
+  asm("v_lshl_add_u32 %1, %3, 1, -1\n\t"
+      "v_lshl_add_u32 %2, %4, 1, -1\n\t"
+      "v_min3_u32 %0, %0, %1, %2\n\t"
+      "v_lshl_add_u32 %1, %5, 1, -1\n\t"
+      "v_lshl_add_u32 %2, %6, 1, -1\n\t"
+      "v_min3_u32 %0, %0, %1, %2"
+      : "+v"(least), "=&v"(t0), "=&v"(t1)
+      : "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     p[q] = make_uint2(pack_bf16(r[0], r[1]), pack_bf16(r[2], r[3]));
@@ -1041,7 +1054,7 @@ __device__ __forceinline__ void split3(const float4& v, uint2 (&p)[3]) {
   }
 }
 template <bool KC, int ROWS>
-__device__ __forceinline__ void split_store(uint16_t* S, const float4 (&v)[ROWS / 64]) {
+__device__ __forceinline__ void split_store(uint16_t* S, const float4 (&v)[ROWS / 64], uint32_t& least) {
   const int t = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < ROWS / 64; ++i) {
@@ -1054,7 +1067,7 @@ __device__ __forceinline__ void split_store(uint16_t* S, const float4 (&v)[ROWS 
       at = k * ROWS + 8 * ((c >> 3) ^ (ROWS == 128 ? 4 * (k & 3) : 2 * (k & 2))) + (c & 4);
     }
     uint2 p[3];
-    split3(v[i], p);
+    split3(v[i], p, least);
 #pragma unroll
     for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(S + q * ROWS * SK + at) = p[q];
   }
@@ -1316,7 +1329,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     }
   } else {
   float ssq = 0.f;  // E_NORMIN: below
-  bool chain = false;  // by the fp32 chain: a sum of the split products is not finite
+  bool chain = false;  // by the fp32 chain: an operand value has no exact split
   float rss[MT] = {};  // E_NORMIN: this thread's sums of squares over rows t / 4 + 64 i
   {
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
@@ -1328,6 +1341,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) lo[i][j][r] = 0.f;
     float4 cs4 = make_float4(0.f, 0.f, 0.f, 0.f);  // E_DBIAS: column sums over the thread's k rows
+    uint32_t least = ~0u;
     struct Regs {
       float4 a[MT], b[2];
     };
@@ -1364,8 +1378,8 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
           R.b[i] = make_float4(R.b[i].x * g, R.b[i].y * g, R.b[i].z * g, R.b[i].w * g);
         }
       }
-      split_store<!TA, BMT>(S16 + st * SPLIT_STG, R.a);
-      split_store<TB, BN>(S16 + st * SPLIT_STG + 3 * BMT * SK, R.b);
+      split_store<!TA, BMT>(S16 + st * SPLIT_STG, R.a, least);
+      split_store<TB, BN>(S16 + st * SPLIT_STG + 3 * BMT * SK, R.b, least);
     };
     // chunk k0 from stage st; R holds chunk k0 + SK and takes chunk k0 + 3 SK
     auto step = [&](int k0, int st, Regs& R) {
@@ -1419,7 +1433,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
         if (k0 + SK < kend) step(k0 + SK, 1, r0);
       }
     }
-    bool bad = false;
+    bool bad = least < kLeastSplit;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -1779,7 +1793,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void ge
 // 64 x 128 tiles for the products whose 128 x 128 tiles would leave each CU fewer than two
 // workgroups (d = 128 outputs over 32K rows): twice the workgroups, half the serial chain each.
 template <bool TA, bool TB, int E>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void gemm_f32_m64_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gemm_f32_m64_kernel(
     GemmArgs p) {
   const int logical = xcd_logical();
   if (logical >= p.nblocks) return;
@@ -1880,7 +1894,7 @@ __device__ __forceinline__ void s_frag(const float* X, int r, int k0, float (&f)
 }
 
 template <bool TA, bool TB, int E>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gemm_small_kernel(GemmArgs p) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void gemm_small_kernel(GemmArgs p) {
   __shared__ __align__(16) float smem[S_SMEM];
   float* const As = smem;
   float* const Bs = smem + S_PANEL;
@@ -1907,7 +1921,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float csum = 0.f;  // E_DBIAS: column t%64 of op(B) over rows 8*(t/64) .. +8 of each panel
-  bool chain = false;
+  bool chain = false;  // (as in gemm_tile)
   {  // the split products (gemm_tile's, a 32 x 32 block a wave)
     constexpr int STG = 3 * (SBM + SBN) * SK;
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
@@ -1915,6 +1929,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
 #pragma unroll
     for (int r = 0; r < 16; ++r) lo[r] = 0.f;
     float4 cs4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    uint32_t least = ~0u;
     struct Regs {
       float4 a[1], b[1];
     };
@@ -1935,8 +1950,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
         cs4.z += in ? R.b[0].z : 0.f;
         cs4.w += in ? R.b[0].w : 0.f;
       }
-      split_store<!TA, SBM>(S16 + st * STG, R.a);
-      split_store<TB, SBN>(S16 + st * STG + 3 * SBM * SK, R.b);
+      split_store<!TA, SBM>(S16 + st * STG, R.a, least);
+      split_store<TB, SBN>(S16 + st * STG + 3 * SBM * SK, R.b, least);
     };
     auto products = [&](int st) {
       bf16x8 fa[3], fb[3];
@@ -1999,7 +2014,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void ge
         if (k0 + SK < kend) step(k0 + SK, 1, r0);
       }
     }
-    bool bad = false;
+    bool bad = least < kLeastSplit;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       acc[r] += lo[r];

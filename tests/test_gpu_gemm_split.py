@@ -1,7 +1,7 @@
 """The fp32 products formed from three-piece bf16 splits (csrc/gemm.hip), at the edges of their paths:
 the 64 x 64, 64 x 128 and 128 x 128 tiles, whole pairs of 16-deep chunks (the branch-free loop) and
 remainders, split K, operands with no bf16 split (infinities, NaN, values past the largest bf16) and
-values whose third piece underflows. Reference: the f64 product of the same fp32 values.
+values whose pieces underflow. Reference: the f64 product of the same fp32 values.
 
 Bounds: the pairs of pieces left out are below 3 * 2^-26 of a term and a 16-deep step rounds its sum a
 few times: 2^-23 (K / 4 + 8) of the sum of |terms| an element. That alone would let a missing pair
@@ -70,12 +70,23 @@ def test_zero_times_infinity():
     assert np.isnan(got[3, 7]) and not np.any(np.isnan(np.delete(got, 3, 0)))
 
 
-@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (10247, 128, 40), (2048, 2048, 32)])
-def test_third_piece_underflows(M, N, K):
-    """Values near 2^-115: an absolute accuracy of 2^-134 a value."""
-    A, B = operands(0, 0, M, N, K)
-    A *= np.float32(2.0**-115)
-    B *= np.float32(2.0**60)
-    got = product(0, 0, A, B).astype(np.float64)
-    ref, mag = exact(0, 0, A, B)
-    assert np.all(np.abs(got - ref) <= 2.0**-23 * (K / 4 + 8) * mag + 2.0**-134 * np.abs(f32(B)).sum(0))
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 66, 40), (60, 70, 1100), (10247, 128, 40), (2048, 2048, 32)])
+@pytest.mark.parametrize("power", [-118, -128])
+def test_third_piece_underflows(tA, tB, M, N, K, power):
+    """Values near 2^-118, whose third piece bf16 cannot hold (2^-134 of an absolute error is 4e-6 of them, as a
+    2-norm), and subnormal ones, whose second it cannot, are multiplied as fp32 values: either operand of
+    them, or one line of it beside zeros. The 2-norm of K independent roundings of partial sums no larger than the
+    result's 2-norm: 2^-24 sqrt(K)."""
+    for small in (0, 1):
+        for one_line in (False, True):
+            X = list(operands(tA, tB, M, N, K))
+            X[small] *= np.float32(2.0**power)
+            X[1 - small] *= np.float32(2.0**60)
+            if one_line:  # the last row of op(A) or column of op(B)
+                line = X[small].T if small != (tA, tB)[small] else X[small]
+                line[:-1] = 0.0
+            got = product(tA, tB, *X).astype(np.float64)
+            ref, mag = exact(tA, tB, *X)
+            assert np.all(np.abs(got - ref) <= 2.0**-23 * (K / 4 + 8) * mag)
+            assert np.linalg.norm(got - ref) <= 2.0**-24 * K**0.5 * np.linalg.norm(ref)
