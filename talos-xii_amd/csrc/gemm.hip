@@ -994,7 +994,9 @@ __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb,
 // (normal operands; 2.0e-7 -> 6.5e-8 and 8.1e-7 -> 2.8e-7 of the result's norm).
 // Values past the largest bf16 (3.39e38) and infinities have no such split: a tile whose sums are
 // not all finite is formed again by the fp32 chain. So is a tile that meets a nonzero value below
-// 2^-110, whose last bits are below bf16's least subnormal, 2^-133.
+// 2^-110, whose last bits are below bf16's least subnormal, 2^-133, and every tile of a product with
+// K = 1, which the chain rounds once (2-norm of the error 1.02x to 1.04x with the pairs left out, from
+// K = 2 on 0.89x and less).
 //
 // Panels of SK = 16 k values a stage, two stages: chunk c is multiplied while chunk c + 1 (in
 // registers, loaded two chunks earlier) is split and stored to the other stage, one barrier a
@@ -1447,7 +1449,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     if (lane == 0) bad_wave[w] = 0;
     if (__any(bad) && lane == 0) bad_wave[w] = 1;
     lds_barrier();
-    chain = (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
+    chain = p.K == 1 || (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
     if constexpr ((E & E_DBIAS) != 0) {
       // the eight row groups' sums of each column, added below as the chain's two halves are
       if (m0 == 0 && !chain) {
@@ -2026,7 +2028,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
     if constexpr ((E & E_DBIAS) != 0)
       if (m0 == 0) *reinterpret_cast<float4*>(smem + (threadIdx.x >> 4) * SBN + 4 * (threadIdx.x & 15)) = cs4;
     lds_barrier();
-    chain = (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
+    chain = p.K == 1 || (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
     if constexpr ((E & E_DBIAS) != 0) {
       // the sixteen k rows' sums of each column, four to a thread, added below as the chain's
       // quarters are

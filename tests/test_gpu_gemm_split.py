@@ -90,3 +90,12 @@ def test_third_piece_underflows(tA, tB, M, N, K, power):
             ref, mag = exact(tA, tB, *X)
             assert np.all(np.abs(got - ref) <= 2.0**-23 * (K / 4 + 8) * mag)
             assert np.linalg.norm(got - ref) <= 2.0**-24 * K**0.5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N", [(64, 64), (70, 33), (10247, 128), (2049, 2047)])
+def test_one_product(tA, tB, M, N):
+    """K = 1: every element is the fp32 product of its two operands, rounded once."""
+    A, B = operands(tA, tB, M, N, 1)
+    a, b = A.reshape(M, 1), B.reshape(1, N)
+    assert np.array_equal(product(tA, tB, A, B), a * b)
