@@ -985,13 +985,14 @@ __device__ __forceinline__ bf16x8 dl_frag_kmaj(const uint16_t* S, int s, int cb,
 // fp32 products on the bf16 matrix cores. Each operand value is split as it is staged into three
 // bf16 pieces, x = x0 + x1 + x2 (each the nearest bf16 to what the earlier ones left: 8 bits a piece
 // and the signs hold the 24 bits of an fp32 exactly), and a product is formed from the six pairs of
-// pieces with index sum <= 2 on v_mfma_f32_32x32x16_bf16; the three pairs left out are below 2^-26
-// of a term. x0 y0 has an accumulator of its own and the five small pairs another, added at the
-// end: with all six in one, each small product is rounded towards minus infinity at the large sum's
-// last bit, a bias that a sum over many splits of K keeps. Six 16-deep products take 192 cycles
-// where eight 2-deep fp32 ones take 512, and a K of 128 has 8 roundings at the sum's size
-// instead of 64: the error against f64 is 0.32x (K = 128) to 0.34x (K = 2048) of the fp32 chain's
-// (normal operands; 2.0e-7 -> 6.5e-8 and 8.1e-7 -> 2.8e-7 of the result's norm).
+// pieces with index sum <= 2 on v_mfma_f32_32x32x16_bf16; the three pairs left out are below 2^-24
+// of a term together (x1 y2 and x2 y1 below 2^-25 each). x0 y0 has an accumulator of its own and
+// the five small pairs another, added at the end: with all six in one, each small product is rounded
+// towards minus infinity at the large sum's last bit, a bias that a sum over many splits of K keeps. Six
+// 16-deep products take 192 cycles where eight 2-deep fp32 ones take 512, and a K of 128 has 8 roundings
+// at the sum's size instead of 64. The 2-norm of the error against f64, fp32 chain -> split: normal
+// operands 2.0e-7 -> 6.5e-8 (K = 128) and 8.1e-7 -> 2.7e-7 (K = 2048), uniform in (0, 1), where every
+// partial sum is large against its next term, 6.0e-7 -> 2.2e-7 (K = 2048) and 1.2e-6 -> 4.2e-7 (K = 8192).
 // Values past the largest bf16 (3.39e38) and infinities have no such split: a tile whose sums are
 // not all finite is formed again by the fp32 chain. So is a tile that meets a nonzero value below
 // 2^-110, whose last bits are below bf16's least subnormal, 2^-133, and every tile of a product with
