@@ -67,10 +67,6 @@ constexpr int NBUF = TALOS_GEMM_DBUF ? 2 : 1;
 #ifndef TALOS_NBPRE_M64
 #define TALOS_NBPRE_M64 0
 #endif
-// Wave priority (s_setprio) of the main loop's products, 0..3 (1: C4 2.398 -> 2.388 ms).
-#ifndef TALOS_GEMM_PRIO
-#define TALOS_GEMM_PRIO 1
-#endif
 
 // Epilogue flags (template parameter E).
 enum : int {
@@ -840,41 +836,14 @@ __device__ __forceinline__ void normb_rows(const GemmArgs& p, const float* T, in
 }
 
 // ---------------------------------------------------------------------------
-// Direct-to-LDS panels (TALOS_GEMM_DLDS; NT products, whose two operands are both k-contiguous,
-// on 128-row tiles: C4 2.361-2.370 -> 2.339 ms; the NN products, whose B panel is k-major, lost
-// more than the NT ones gained, 235 -> 242 and 205 -> 219 us at C4): interior tiles stream their panels straight from global memory into LDS with
-// global_load_lds_dwordx4 (no register staging, no LDS store instructions), DK = 16 k a chunk in
-// two LDS stages. A wave's load writes 1 KB of consecutive LDS (16 bytes a lane), so the panels
-// X[r][k] (16 floats a row, 16 rows a 1 KB block) are unpadded and their 16-byte pieces permuted
-// instead, by choosing which global piece each lane fetches: piece p of row r sits in slot
-// p ^ ((r >> 2) & 3), so the 16 rows one fragment read spans fall on 16 distinct bank groups.
+// Direct-to-LDS panels of the bf16 copies (TALOS_GEMM_DLDS): interior tiles stream their panels
+// straight from global memory into LDS with global_load_lds_dwordx4 (no register staging, no LDS store
+// instructions). A wave's load writes 1 KB of consecutive LDS (16 bytes a lane), so the panels are unpadded
+// and their 16-byte pieces permuted instead, by choosing which global piece each lane fetches.
 // ---------------------------------------------------------------------------
 #ifndef TALOS_GEMM_DLDS
 #define TALOS_GEMM_DLDS 1
 #endif
-constexpr int DK = 16;
-// The ROWS-row panel of X (k-contiguous rows of pitch ld) at rows r0.., k0.. into S: block b
-// (rows 16 b .. 16 b + 15) by wave b % 4
-template <int ROWS>
-__device__ __forceinline__ void dl_panel(const float* __restrict__ X, long long ld, int r0, int k0, float* S) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int blk = w; blk < ROWS / 16; blk += 4) {
-    const int row = 16 * blk + (lane >> 2), piece = (lane & 3) ^ ((row >> 2) & 3);
-    __builtin_amdgcn_global_load_lds(X + (long long)(r0 + row) * ld + k0 + 4 * piece, S + 256 * blk, 16, 0, 0);
-  }
-}
-// row r's (and, TWO, row r + 32's) values at k = k0 .. k0 + 3 of a direct-load panel
-template <bool TWO>
-__device__ __forceinline__ void dl_frag(const float* X, int r, int k0, float (&f0)[4], float (&f1)[4]) {
-  const int o = 4 * ((k0 >> 2) ^ ((r >> 2) & 3));  // rows r and r + 32 share the permutation
-  const float4 v0 = *reinterpret_cast<const float4*>(X + r * DK + o);
-  f0[0] = v0.x; f0[1] = v0.y; f0[2] = v0.z; f0[3] = v0.w;
-  if (TWO) {
-    const float4 v1 = *reinterpret_cast<const float4*>(X + (r + 32) * DK + o);
-    f1[0] = v1.x; f1[1] = v1.y; f1[2] = v1.z; f1[3] = v1.w;
-  }
-}
 
 // The bf16 copies' k-contiguous 128-row panels (rows of BKB = 64 bf16, 128 bytes: eight rows a
 // 1 KB block) straight into LDS; piece p (8 values) of row r sits in slot p ^ ((r >> 1) & 7), so
@@ -1093,7 +1062,7 @@ __device__ __forceinline__ void split_products(const uint16_t* S, int ra, int rb
 #pragma unroll
     for (int x = 0; x < 2; ++x) b[x][q] = split_frag<KB>(Sb + q * 128 * SK, rb + 32 * x, lane);
 #pragma unroll
-    for (int x = 0; x < MT; ++x) a[x][q] = split_frag<KA>(S + q * AROWS * SK, ra + 32 * x, lane);
+    for (int x = 0; x < MT; ++x) a[x][q] = split_frag<KA, AROWS>(S + q * AROWS * SK, ra + 32 * x, lane);
   }
   auto add = [&](int pa, int pb, floatx16 (&c)[MT][2]) {
 #pragma unroll
@@ -1501,9 +1470,6 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     }
     const float* Ap = Abase + buf * PANEL;
     const float* Bp = Bbase + buf * PANEL;
-    // the chunk's products at a raised wave priority: a wave with products ready issues ahead of
-    // the waves of the CU's other workgroups that are storing panels or waiting at the barrier
-    __builtin_amdgcn_s_setprio(TALOS_GEMM_PRIO);
 #pragma unroll
     for (int j = 0; j < BK / 8; ++j) {
       // fragments of steps 4j .. 4j+3: k = 8j + 4h + q for q = 0..3
@@ -1523,7 +1489,6 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
         }
       }
     }
-    __builtin_amdgcn_s_setprio(0);
     if constexpr ((E & E_DBIAS) != 0) {
       // column sums of the B panel Bs[k][n] (k-major): thread t sums column t%128 over half the rows
       if (m0 == 0) {
