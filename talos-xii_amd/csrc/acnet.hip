@@ -62,7 +62,7 @@ struct Smem {
   float C[T * LC];                  // [c | k_r], later their gradients
   float St[T * LS];                 // states | 1
   float P[T * H], S[T * H], rs[T];  // probabilities, dL/dscore, rstd
-  float We[IN * D], be[D], g1[D];   // (be read as row IN of We)
+  float We[(IN + 1) * D], g1[D];    // (row IN of We: its bias)
   float Q[GS * LQ];                 // [q_c | q_r]
   float QA[GS * LH];                // W_uk_h q_c; later the query path's dL/dxn
   float Z[GS * LH];                 // sum_j p_j c_j
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
     }
   }
   sm.We[tid] = P[oWE + tid];  // IN * D = NTHR
-  if (tid < D) sm.be[tid] = P[oBE + tid];
+  if (tid < D) sm.We[IN * D + tid] = P[oBE + tid];
   if (tid < D) sm.g1[tid] = P[oG1 + tid];
   static_assert(IN * D == NTHR, "one embedding weight a thread");
 
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2))) vo
       keys(w >> 2, 2 * (w & 3), std::integral_constant<int, 2>{});
     }
     {
-      float v = sm.be[lane];
+      float v = sm.We[IN * D + lane];
       const float* st = sm.St + sm.lrow[w] * LS;
 #pragma unroll
       for (int f = 0; f < IN; ++f) v = fmaf(st[f], sm.We[f * D + lane], v);
