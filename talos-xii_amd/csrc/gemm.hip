@@ -1301,9 +1301,9 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     }
   } else {
   float ssq = 0.f;  // E_NORMIN: below
-  bool chain = false;  // by the fp32 chain: an operand value has no exact split
+  bool chain = p.K == 1;  // by the fp32 chain: so is a tile with an operand value that has no exact split
   float rss[MT] = {};  // E_NORMIN: this thread's sums of squares over rows t / 4 + 64 i
-  {
+  if (!chain) {
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
     floatx16 lo[MT][2];
 #pragma unroll
@@ -1419,7 +1419,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     if (lane == 0) bad_wave[w] = 0;
     if (__any(bad) && lane == 0) bad_wave[w] = 1;
     lds_barrier();
-    chain = p.K == 1 || (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
+    chain = (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
     if constexpr ((E & E_DBIAS) != 0) {
       // the eight row groups' sums of each column, added below as the chain's two halves are
       if (m0 == 0 && !chain) {
@@ -1472,6 +1472,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
     const float* Bp = Bbase + buf * PANEL;
 #pragma unroll
     for (int j = 0; j < BK / 8; ++j) {
+      if (k0 + 8 * j >= kend) break;
       // fragments of steps 4j .. 4j+3: k = 8j + 4h + q for q = 0..3
       float fa0[4], fa1[4], fb0[4], fb1[4];
       if constexpr (MT == 2)
@@ -1889,8 +1890,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float csum = 0.f;  // E_DBIAS: column t%64 of op(B) over rows 8*(t/64) .. +8 of each panel
-  bool chain = false;  // (as in gemm_tile)
-  {  // the split products (gemm_tile's, a 32 x 32 block a wave)
+  bool chain = p.K == 1;  // (as in gemm_tile)
+  if (!chain) {  // the split products (gemm_tile's, a 32 x 32 block a wave)
     constexpr int STG = 3 * (SBM + SBN) * SK;
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
     floatx16 lo;
@@ -1994,7 +1995,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
     if constexpr ((E & E_DBIAS) != 0)
       if (m0 == 0) *reinterpret_cast<float4*>(smem + (threadIdx.x >> 4) * SBN + 4 * (threadIdx.x & 15)) = cs4;
     lds_barrier();
-    chain = p.K == 1 || (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
+    chain = (bad_wave[0] | bad_wave[1] | bad_wave[2] | bad_wave[3]) != 0;
     if constexpr ((E & E_DBIAS) != 0) {
       // the sixteen k rows' sums of each column, four to a thread, added below as the chain's
       // quarters are
@@ -2029,6 +2030,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
     if (more) load(k0 + BK);
 #pragma unroll
     for (int j = 0; j < BK / 8; ++j) {
+      if (k0 + 8 * j >= kend) break;
       float fa[4], fb[4];
       s_frag<!TA>(As, wm * 32 + l32, 8 * j + 4 * h, fa);
       s_frag<TB>(Bs, wn * 32 + l32, 8 * j + 4 * h, fb);
