@@ -1363,12 +1363,13 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
       lds_barrier();
     };
     Regs r0, r1;
-    if (interior && kbeg < kend && (kend - kbeg) % (2 * SK) == 0) {
-      // whole chunks, an even number: no branch inside a step, so that the split of the next chunk and its stores can
-      // be issued between the products (a branch there made a wave walk its products, then its
-      // split: 2430 cycles a chunk against the products' 1536 for two waves a SIMD), nor around the
-      // first loads (the wait before a split would then drain the loads issued after its own). The
-      // last steps split and store registers nobody reads and load the last chunk again.
+    if (interior && kend - kbeg > 2 * SK && (kend - kbeg) % (2 * SK) == 0) {
+      // whole chunks, an even number, more than two (this loop would load five for two: 65536 x 2048 x
+      // 32 154 -> 132 us by the other): no branch inside a step, so that the split of the next chunk
+      // and its stores can be issued between the products (a branch there made a wave walk its
+      // products, then its split: 2430 cycles a chunk against the products' 1536 for two waves a SIMD),
+      // nor around the first loads (the wait before a split would then drain the loads issued after
+      // its own). The last steps split and store registers nobody reads and load the last chunk again.
       auto fetch = [&](int k0, Regs& R) {
         const int kn = min(k0, kend - SK);
         split_load<!TA, false, BMT>(A, p.lda, m0, p.M, kn, kend, true, R.a);
@@ -1939,7 +1940,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
       lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[2], fb[0], lo, 0, 0, 0);
     };
     Regs r0, r1;
-    if (interior && kbeg < kend && (kend - kbeg) % (2 * SK) == 0) {
+    if (interior && kend - kbeg > 2 * SK && (kend - kbeg) % (2 * SK) == 0) {
       auto fetch = [&](int k0, Regs& R) {
         const int kn = min(k0, kend - SK);
         split_load<!TA, false, SBM>(A, p.lda, m0, p.M, kn, kend, true, R.a);
@@ -2429,10 +2430,14 @@ static int num_cus();
 // split-K decision): 64 when the output is one tile wide, the 128-row tiles would give fewer
 // than two workgroups per CU, K is not split and the 64-row kernel is instantiated for e
 // (measured at 32768 rows: the norm-backward products 61 -> 56 us at K = 512 and 41 -> 36 us at
-// K = 256; with 1024 or more tiles the 128-row tiles are 3-12% faster).
+// K = 256; with 1024 or more tiles the 128-row tiles are 3-12% faster). At any width for K of at
+// most two split chunks, where a tile is mostly its epilogue: four workgroups a CU store beside
+// each other's loads where the 128-row tiles have two (K = 8, plain: 65536 x 2048 127 -> 108 us,
+// 65536 x 1024 65 -> 60, 16384 x 2048 32 -> 24, 8192 x 2048 18.4 -> 15.1; K = 64 gains nothing).
 static int tile_rows(const GemmDesc& d, int e, int ksplit) {
   const long long tiles = (long long)((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN) * d.batch;
-  if (d.bf16 || d.batch != 1 || d.N > BN || ksplit > 1) return BM;
+  if (d.bf16 || d.batch != 1 || ksplit > 1) return BM;
+  if (d.N > BN) return d.K <= 2 * SK && pick_m64(d.transA != 0, d.transB != 0, e) ? 64 : BM;
   if (tiles >= 2LL * num_cus() && !(TALOS_NBPRE_M64 && (e & E_NBPRE) != 0)) return BM;
   return pick_m64(d.transA != 0, d.transB != 0, e) ? 64 : BM;
 }

@@ -1,6 +1,6 @@
 """The fp32 products formed from three-piece bf16 splits (csrc/gemm.hip), at the edges of their paths:
 the 64 x 64, 64 x 128 and 128 x 128 tiles, whole pairs of 16-deep chunks (the branch-free loop) and
-remainders, split K, operands with no bf16 split (infinities, NaN, values past the largest bf16) and
+remainders, split K, K of one or two chunks, operands with no bf16 split (infinities, NaN, values past the largest bf16) and
 values whose pieces underflow. Reference: the f64 product of the same fp32 values.
 
 Bounds: the pairs of pieces left out are below 2^-24 of a term (2^-25 each of the two larger ones) and a
@@ -41,7 +41,9 @@ def exact(tA, tB, A, B):
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(64, 64, 32), (65, 63, 16), (1, 64, 17), (130, 96, 48), (60, 70, 5003),  # 64 x 64
                                    (10240, 128, 64), (10247, 128, 40), (10300, 65, 31),  # 64 x 128
-                                   (2048, 2048, 32), (2049, 2047, 48), (2100, 2048, 33)])  # 128 x 128
+                                   (2048, 2048, 32), (2049, 2047, 48), (2100, 2048, 33),  # 128 x 128
+                                   (2048, 2048, 64), (2049, 2047, 16), (2049, 2047, 17), (2112, 2048, 31)])
+# (of the last two lines K <= 32 with A plain: 64 x 128, the width of several tiles)
 def test_split_products(tA, tB, M, N, K):
     A, B = operands(tA, tB, M, N, K)
     got = product(tA, tB, A, B).astype(np.float64)
@@ -50,7 +52,7 @@ def test_split_products(tA, tB, M, N, K):
     assert np.linalg.norm(got - ref) <= 5e-7 * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 64, 40), (10247, 128, 32), (2049, 2048, 32)])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 64, 40), (10247, 128, 32), (2049, 2048, 32), (2049, 2048, 64)])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38, -3.4e38])
 def test_values_without_a_split(M, N, K, value):
     A, B = operands(0, 0, M, N, K)
@@ -93,7 +95,8 @@ def test_zero_times_infinity():
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 66, 40), (60, 70, 1100), (10247, 128, 40), (2048, 2048, 32)])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 66, 40), (60, 70, 1100), (10247, 128, 40), (2048, 2048, 32),
+                                   (2048, 2048, 64)])
 @pytest.mark.parametrize("power", [-118, -128])
 def test_third_piece_underflows(tA, tB, M, N, K, power):
     """Values near 2^-118, whose third piece bf16 cannot hold (2^-134 of an absolute error is 4e-6 of them, as a
