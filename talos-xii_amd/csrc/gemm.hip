@@ -2290,14 +2290,17 @@ static int epi_flags(const GemmDesc& d) {
 // and split K instead, which reads each operand half as often.
 static void (*pick_m64(bool tA, bool tB, int e))(GemmArgs);
 // The 64 x 64 tile kernel for products of fewer 128 x 128 tiles than CUs and at most 2^30 MACs;
-// not for one 128-wide column of tiles over at least 40 rows a CU where the 64 x 128 tiles are
-// instantiated: these split half as many operand values a product, and their norm epilogues save
-// the row kernels (14700 x 128 x 512: 230 workgroups, about one a CU, against 460).
+// not for one column of tiles, 65 to 128 wide, over many rows where the 64 x 128 tiles are instantiated:
+// from 40 rows a CU with a row norm in the epilogue, which saves the row kernels (minibatch of 1000 x 14
+// tokens 577 -> 553 us, 650 x 16 515 -> 503), from 64 rows a CU without (at 40 the three products of a
+// 12800 x 512 x 100 Linear took 91 us against 82). Up to 64 columns half of a 128-wide tile
+// is padding: 64 x 64 tiles at any height (20011 x 64 x 512 52 -> 27 us, 16384 x 8 x 64 7.9 -> 6.4).
 static bool use_small(const GemmDesc& d, int num_cu) {
   const long long tiles = (long long)((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN) * d.batch;
   const double macs = (double)d.M * d.N * d.K * d.batch;
-  if (!d.bf16 && d.batch == 1 && d.N <= BN && d.N > SBN && d.M >= 40 * num_cu && !d.transA && d.ksplit <= 1 &&
-      pick_m64(false, d.transB != 0, epi_flags(d)) != nullptr)
+  const int e = epi_flags(d);
+  if (!d.bf16 && d.batch == 1 && d.N <= BN && d.N > SBN && d.M >= ((e & (E_NORM | E_NORMB)) ? 40 : 64) * num_cu &&
+      !d.transA && d.ksplit <= 1 && pick_m64(false, d.transB != 0, e) != nullptr)
     return false;  // one 128-wide column of tiles over many rows: the 64-row tiles
   return !d.bf16 && d.cmap_w == 0 && !d.rd_D && tiles < num_cu && macs <= 1073741824.0;
 }
