@@ -22,6 +22,7 @@ import re
 def short(name):
     """'void talos::gemm_f32_kernel<true, false, 768>(talos::GemmArgs)' -> 'gemm_f32_kernel<true, false, 768>'."""
     n = re.sub(r"^void ", "", name)
+    n = n.replace("(anonymous namespace)::", "")
     n = re.sub(r"^talos::", "", n)
     depth, out = 0, []
     for ch in n:
