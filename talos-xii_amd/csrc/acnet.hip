@@ -19,8 +19,8 @@
 // row; acnet_reduce_kernel adds the rows in a fixed order in f64.
 //
 // Bound by the latency of its 28 dependent phases (LDS round trips and barriers, one workgroup per
-// CU: 160 KB of LDS; about 95 k cycles a group of 8 samples x 16 tokens, 25 k of them in the four
-// token-product phases, which run at about half of the fp32 matrix rate), then by the partial rows
+// CU: 160 KB of LDS; about 93 k cycles a group of 8 samples x 16 tokens, the matrix pipe busy for a
+// third of them; 256 samples leave three quarters of the CUs idle), then by the partial rows
 // (181 KB a workgroup). One MI355X, minibatch forward + backward: 4096 x 16 tokens 849 -> 87 us,
 // 256 ragged samples of up to 16 tokens 411 -> 39 us.
 #include "acnet.hpp"
