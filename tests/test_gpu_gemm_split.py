@@ -40,7 +40,8 @@ def exact(tA, tB, A, B):
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(64, 64, 32), (65, 63, 16), (1, 64, 17), (130, 96, 48), (60, 70, 5003),  # 64 x 64
-                                   (10240, 128, 64), (10247, 128, 40), (10300, 65, 31),  # 64 x 128
+                                   (10240, 128, 64), (10247, 128, 40), (10300, 65, 31), (16383, 128, 33),
+                                   (16384, 128, 64), (16391, 128, 40), (16400, 65, 31),  # 64 x 128 (tA = 0)
                                    (2048, 2048, 32), (2049, 2047, 48), (2100, 2048, 33),  # 128 x 128
                                    (2048, 2048, 64), (2049, 2047, 16), (2049, 2047, 17), (2112, 2048, 31)])
 # (of the last two lines K <= 32 with A plain: 64 x 128, the width of several tiles)
@@ -52,7 +53,8 @@ def test_split_products(tA, tB, M, N, K):
     assert np.linalg.norm(got - ref) <= 5e-7 * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 64, 40), (10247, 128, 32), (2049, 2048, 32), (2049, 2048, 64)])
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 64, 40), (10247, 128, 32), (16391, 128, 32), (2049, 2048, 32),
+                                   (2049, 2048, 64)])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38, -3.4e38])
 def test_values_without_a_split(M, N, K, value):
     A, B = operands(0, 0, M, N, K)
@@ -67,7 +69,7 @@ def test_values_without_a_split(M, N, K, value):
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(70, 64, 40), (60, 70, 1100), (10247, 128, 40), (2049, 2047, 48), (150, 130, 70000)])
+@pytest.mark.parametrize("M,N,K", [(70, 64, 40), (60, 70, 1100), (16391, 128, 40), (2049, 2047, 48), (150, 130, 70000)])
 def test_infinity_in_any_layout(tA, tB, M, N, K):
     """One infinity in the last line of either operand: that line of C infinite, every other element as finite ones
     are (tiles without one by the split products, the line's tiles, in one K split of the long ones, by fp32 products:
@@ -95,7 +97,7 @@ def test_zero_times_infinity():
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 66, 40), (60, 70, 1100), (10247, 128, 40), (2048, 2048, 32),
+@pytest.mark.parametrize("M,N,K", [(64, 64, 32), (70, 66, 40), (60, 70, 1100), (16391, 128, 40), (2048, 2048, 32),
                                    (2048, 2048, 64)])
 @pytest.mark.parametrize("power", [-118, -128])
 def test_third_piece_underflows(tA, tB, M, N, K, power):
@@ -118,7 +120,7 @@ def test_third_piece_underflows(tA, tB, M, N, K, power):
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N", [(64, 64), (70, 33), (10247, 128), (2049, 2047)])
+@pytest.mark.parametrize("M,N", [(64, 64), (70, 33), (16391, 128), (2049, 2047)])
 def test_one_product(tA, tB, M, N):
     """K = 1: every element is the fp32 product of its two operands, rounded once."""
     A, B = operands(tA, tB, M, N, 1)
@@ -200,7 +202,7 @@ def test_policy_by_fp32_products(B, S):
     check_same(got[1:], ref[1:], (slices, None, None))
 
 
-@pytest.mark.parametrize("M,N", [(64, 64), (10247, 128), (2048, 2048)])
+@pytest.mark.parametrize("M,N", [(64, 64), (16391, 128), (2048, 2048)])
 @pytest.mark.parametrize("K", [16, 40, 512])
 def test_largest_left_out_pairs(M, N, K):
     """1 + 2^-8 - 2^-17 = 1, 2^-8, -2^-17 in pieces: the pairs left out come to 3.97 * 2^-26 of each term, all of one
@@ -212,7 +214,7 @@ def test_largest_left_out_pairs(M, N, K):
 
 
 @pytest.mark.parametrize("draw", ["uniform", "normal", "absolute"])
-@pytest.mark.parametrize("M,N,K", [(64, 64, 512), (10240, 128, 512), (4096, 4096, 512), (4096, 4096, 2048),
+@pytest.mark.parametrize("M,N,K", [(64, 64, 512), (16384, 128, 512), (4096, 4096, 512), (4096, 4096, 2048),
                                    (4096, 4096, 8192)])  # (K in one piece)
 def test_no_less_accurate_than_fp32_products(M, N, K, draw):
     """Sums that grow with every term as well as zero-mean ones: the 2-norm of the error against that of the fp32
