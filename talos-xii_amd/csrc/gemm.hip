@@ -1303,7 +1303,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
   float ssq = 0.f;  // E_NORMIN: below
   bool chain = p.K == 1;  // by the fp32 chain: so is a tile with an operand value that has no exact split
   float rss[MT] = {};  // E_NORMIN: this thread's sums of squares over rows t / 4 + 64 i
-  if (!chain) {
+  if (__builtin_expect(!chain, 1)) {
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
     floatx16 lo[MT][2];
 #pragma unroll
@@ -1432,7 +1432,7 @@ __device__ __forceinline__ void gemm_tile(GemmArgs p, int logical) {
       }
     }
   }
-  if (chain) {
+  if (__builtin_expect(chain, 0)) {  // (out of line: 1000 x 500 x 700 109.5 -> 107.6 us, three products)
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -1892,7 +1892,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float csum = 0.f;  // E_DBIAS: column t%64 of op(B) over rows 8*(t/64) .. +8 of each panel
   bool chain = p.K == 1;  // (as in gemm_tile)
-  if (!chain) {  // the split products (gemm_tile's, a 32 x 32 block a wave)
+  if (__builtin_expect(!chain, 1)) {  // the split products (gemm_tile's, a 32 x 32 block a wave)
     constexpr int STG = 3 * (SBM + SBN) * SK;
     uint16_t* const S16 = reinterpret_cast<uint16_t*>(smem);
     floatx16 lo;
@@ -2007,7 +2007,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void ge
       lds_barrier();
     }
   }
-  if (chain) {
+  if (__builtin_expect(chain, 0)) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float4 ra[2], rb[2];
